@@ -17,7 +17,10 @@
 //   n <= 256 : blocked right-looking LU, one workgroup per matrix
 //              (getrf_blocked.hip, lu_blocked.h): 32-column panels factored in
 //              registers, trailing updates on the FP32 matrix instruction.
-//   n > 256  : one workgroup per matrix working in global memory (L2), with
+//   n <= 2048: blocked over many workgroups per matrix, one launch per 32
+//              columns (getrf_large.hip): a panel holds at most two rows per
+//              thread of one workgroup in registers, which ends at 2048 rows.
+//   n > 2048 : one workgroup per matrix working in global memory (L2), with
 //              explicit row swaps.
 // The n <= 64 and n > 256 paths perform, element by element, the same
 // operations in the same order (l = a_ik / p, a_ij = fma(-l, u_kj, a_ij)) and
@@ -36,7 +39,7 @@ namespace {
 using dev::kWave;
 
 // ---------------------------------------------------------------------------
-// n > 256: one workgroup per matrix, in global memory
+// n > 2048: one workgroup per matrix, in global memory
 // ---------------------------------------------------------------------------
 constexpr int kGlobalThreads = 1024;
 
@@ -139,6 +142,8 @@ void LaunchGetrf(const _aclblas_handle* h, float* const* A, int n, int lda, int*
     } else if (n <= 256) {
         const int cus = h->cu_count > 0 ? h->cu_count : 256;
         LaunchGetrfBlocked<PIVOT>(st, A, n, lda, ipiv, info, batch, batch < 2 * cus ? batch : 2 * cus);
+    } else if (n <= kMaxLargeN) {
+        LaunchGetrfLarge<PIVOT>(st, A, n, lda, ipiv, info, batch);
     } else {
         hipLaunchKernelGGL((GetrfGlobalKernel<PIVOT>), dim3(batch), dim3(kGlobalThreads), 0, st, A, n, lda, ipiv,
                            info, batch);

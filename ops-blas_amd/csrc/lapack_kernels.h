@@ -20,6 +20,11 @@ void LaunchGetrfWaveOutOfPlace(hipStream_t st, const float* const* A, int n, int
 template <bool PIVOT>
 void LaunchGetrfBlocked(hipStream_t st, float* const* A, int n, int lda, int* ipiv, int* info, int batch, int grid);
 
+// LU, 256 < n <= kMaxLargeN, blocked over many workgroups per matrix (getrf_large.hip)
+constexpr int kMaxLargeN = 2048;
+template <bool PIVOT>
+void LaunchGetrfLarge(hipStream_t st, float* const* A, int n, int lda, int* ipiv, int* info, int batch);
+
 // Triangular solves, n <= 64 (getrs_small.hip); false when the shape is not covered.
 bool LaunchGetrsSmall(hipStream_t st, bool trans, int n, int nrhs, const float* const* A, int lda, const int* piv,
                       float* const* B, int ldb, int batch);

@@ -8,8 +8,11 @@
 // getri_batched_kernel.cpp:39-308 (C = I, P, L^-1, U^-1; info = j+1 for the zero
 // u_jj with the largest j).
 //
-// MI355X design.  One workgroup per (system, chunk of right-hand sides).  The
-// chunk of B lives in LDS for the whole solve, already permuted.  Each
+// Orders up to 64 run the register kernels (getrs_small.hip, getri_small.hip),
+// orders up to 2048 the tile kernel (getrs_tile.hip); the kernel here takes
+// the larger ones, whose unknowns times 16 right-hand sides would not fit in
+// LDS.  One workgroup per (system, chunk of right-hand sides).  The chunk of B
+// lives in LDS for the whole solve, already permuted.  Each
 // triangular solve runs in 64-row blocks: wave 0 solves the 64x64 diagonal
 // block with one lane per row (the solved value broadcast by v_readlane, no
 // barriers inside the block), then all waves apply the block to the remaining
@@ -29,7 +32,7 @@ using dev::kWave;
 
 constexpr int kBlk = 64;            // rows per diagonal block
 constexpr int kChunk = 8;           // entries of a trailing row loaded together
-constexpr int kMaxRc = 8;           // right-hand sides per workgroup
+constexpr int kMaxRc = 4;           // right-hand sides per workgroup
 constexpr size_t kLdsBudget = 64 * 1024;
 
 enum SolveMode { kModeN = 0, kModeT = 1, kModeInv = 2 };
@@ -40,41 +43,18 @@ enum SolveMode { kModeN = 0, kModeT = 1, kModeInv = 2 };
 __device__ void BuildPerm(int* perm, int* scratch, const int* piv, int n)
 {
     const int t = threadIdx.x;
-    if (n <= kWave) {
-        if (t < kWave) {
-            const int myp = t < n ? piv[t] - 1 : -1;
-            int src = t;
-            for (int k = 0; k < n; ++k) {
-                const int p = __builtin_amdgcn_readlane(myp, k);
-                if (p >= 0 && p < n && p != k) {
-                    const int sk = __builtin_amdgcn_readlane(src, k);
-                    const int sp = __builtin_amdgcn_readlane(src, p);
-                    if (t == k) {
-                        src = sp;
-                    }
-                    if (t == p) {
-                        src = sk;
-                    }
-                }
-            }
-            if (t < n) {
-                perm[t] = src;
-            }
-        }
-    } else {
-        for (int i = t; i < n; i += blockDim.x) {
-            perm[i] = i;
-            scratch[i] = piv[i] - 1;
-        }
-        __syncthreads();
-        if (t == 0) {
-            for (int k = 0; k < n; ++k) {
-                const int p = scratch[k];
-                if (p >= 0 && p < n && p != k) {
-                    const int x = perm[k];
-                    perm[k] = perm[p];
-                    perm[p] = x;
-                }
+    for (int i = t; i < n; i += blockDim.x) {
+        perm[i] = i;
+        scratch[i] = piv[i] - 1;
+    }
+    __syncthreads();
+    if (t == 0) {
+        for (int k = 0; k < n; ++k) {
+            const int p = scratch[k];
+            if (p >= 0 && p < n && p != k) {
+                const int x = perm[k];
+                perm[k] = perm[p];
+                perm[p] = x;
             }
         }
     }
@@ -335,7 +315,7 @@ __global__ __launch_bounds__(256) void SolveKernel(
     }
 }
 
-// Right-hand sides per workgroup: up to 8, fewer when the LDS chunk would not
+// Right-hand sides per workgroup: up to 4, fewer when the LDS chunk would not
 // fit in 64 KiB.  0 means n is too large.
 int ChooseRc(int n, int nrhs)
 {
@@ -354,7 +334,7 @@ void LaunchSolveRc(hipStream_t st, const float* const* A, int n, int lda, const 
 {
     const int chunks = (nrhs + RC - 1) / RC;
     const size_t lds = static_cast<size_t>(n) * sizeof(int) + static_cast<size_t>(n) * RC * sizeof(float);
-    const int threads = n <= kWave ? kWave : 256;
+    const int threads = 256;
     const dim3 grid(static_cast<unsigned>(static_cast<long long>(batch) * chunks));
     hipLaunchKernelGGL((SolveKernel<RC, MODE>), grid, dim3(threads), lds, st, A, n, lda, piv, B, ldb, nrhs, chunks,
                        info);
@@ -368,16 +348,8 @@ void LaunchSolve(hipStream_t st, int rc, const float* const* A, int n, int lda, 
         case 1: LaunchSolveRc<MODE, 1>(st, A, n, lda, piv, B, ldb, nrhs, info, batch); break;
         case 2: LaunchSolveRc<MODE, 2>(st, A, n, lda, piv, B, ldb, nrhs, info, batch); break;
         case 3: LaunchSolveRc<MODE, 3>(st, A, n, lda, piv, B, ldb, nrhs, info, batch); break;
-        case 4: LaunchSolveRc<MODE, 4>(st, A, n, lda, piv, B, ldb, nrhs, info, batch); break;
-        default: LaunchSolveRc<MODE, 8>(st, A, n, lda, piv, B, ldb, nrhs, info, batch); break;
+        default: LaunchSolveRc<MODE, 4>(st, A, n, lda, piv, B, ldb, nrhs, info, batch); break;
     }
-}
-
-int RoundRc(int rc)
-{
-    if (rc >= 8) return 8;
-    if (rc >= 4) return 4;
-    return rc;
 }
 
 // reference sgetrs_batched_host.cpp:29-40: LAPACK argument positions
@@ -465,14 +437,22 @@ aclblasStatus_t GetrsBatchedLaunch(hipStream_t st, bool trans, int n, int nrhs, 
     if (LaunchGetrsSmall(st, trans, n, nrhs, A, lda, piv, B, ldb, batch)) {
         return LaunchStatus("aclblasSgetrsBatched");
     }
+    if (n <= kMaxTileN) {
+        if (trans) {
+            LaunchSolveTile<kSolveT>(st, n, nrhs, A, lda, piv, B, ldb, nullptr, batch);
+        } else {
+            LaunchSolveTile<kSolveN>(st, n, nrhs, A, lda, piv, B, ldb, nullptr, batch);
+        }
+        return LaunchStatus("aclblasSgetrsBatched");
+    }
     const int rc = ChooseRc(n, nrhs);
     if (rc <= 0) {
         return ACLBLAS_STATUS_NOT_SUPPORTED;
     }
     if (trans) {
-        LaunchSolve<kModeT>(st, RoundRc(rc), A, n, lda, piv, B, ldb, nrhs, nullptr, batch);
+        LaunchSolve<kModeT>(st, rc, A, n, lda, piv, B, ldb, nrhs, nullptr, batch);
     } else {
-        LaunchSolve<kModeN>(st, RoundRc(rc), A, n, lda, piv, B, ldb, nrhs, nullptr, batch);
+        LaunchSolve<kModeN>(st, rc, A, n, lda, piv, B, ldb, nrhs, nullptr, batch);
     }
     return LaunchStatus("aclblasSgetrsBatched");
 }
@@ -483,11 +463,15 @@ aclblasStatus_t GetriBatchedLaunch(hipStream_t st, int n, const float* const* A,
     if (LaunchGetriSmall(st, n, A, lda, piv, C, ldc, info, batch)) {
         return LaunchStatus("aclblasSgetriBatched");
     }
+    if (n <= kMaxTileN) {
+        LaunchSolveTile<kSolveInv>(st, n, n, A, lda, piv, C, ldc, info, batch);
+        return LaunchStatus("aclblasSgetriBatched");
+    }
     const int rc = ChooseRc(n, n);
     if (rc <= 0) {
         return ACLBLAS_STATUS_NOT_SUPPORTED;
     }
-    LaunchSolve<kModeInv>(st, RoundRc(rc), A, n, lda, piv, C, ldc, n, info, batch);
+    LaunchSolve<kModeInv>(st, rc, A, n, lda, piv, C, ldc, n, info, batch);
     return LaunchStatus("aclblasSgetriBatched");
 }
 

@@ -29,6 +29,15 @@ void LaunchGetrfLarge(hipStream_t st, float* const* A, int n, int lda, int* ipiv
 bool LaunchGetrsSmall(hipStream_t st, bool trans, int n, int nrhs, const float* const* A, int lda, const int* piv,
                       float* const* B, int ldb, int batch);
 
+// Triangular solves (op N / T) and inverses of orders 65..kMaxTileN, 16
+// right-hand sides per workgroup (getrs_tile.hip); the bound is the tiles'
+// LDS: 64 bytes per row and 12 for the permutation, 152 KiB at 2048.
+constexpr int kMaxTileN = 2048;
+enum SolveTileMode { kSolveN = 0, kSolveT = 1, kSolveInv = 2 };
+template <SolveTileMode MODE>
+void LaunchSolveTile(hipStream_t st, int n, int nrhs, const float* const* A, int lda, const int* piv, float* const* B,
+                     int ldb, int* info, int batch);
+
 // Inverse C = A^-1 from LU factors, n <= 64 (getrs_small.hip): info[b] = j+1
 // for the zero u_jj with the largest j; false when the shape is not covered.
 bool LaunchGetriSmall(hipStream_t st, int n, const float* const* A, int lda, const int* piv, float* const* C,

@@ -30,6 +30,7 @@
 #include "internal.h"
 #include "lapack_kernels.h"
 #include "lds_dma.h"
+#include "tile16.h"
 
 namespace aclblas {
 namespace {
@@ -40,7 +41,7 @@ constexpr int kT = 16;        // tile order and right-hand sides per workgroup
 constexpr int kSwaps = 64;    // interchanges composed per step of the permutation
 constexpr int kAheadTiles = 4;  // tiles of a wave whose operands are loaded a phase ahead
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+using f32x4 = dev::F32x4;
 
 // Unknown (row, rhs) in LDS: rows of 16, each quad of rows rotated by its own
 // number, so that both a quarter-wave's four consecutive rows (matrix operand)
@@ -48,17 +49,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ int XOff(int row, int rhs)
 {
     return ((row & ~3) + ((row + (row >> 2)) & 3)) * kT + rhs;
-}
-
-// The value of lane group g (16 lanes) in every group.
-template <int g>
-__device__ __forceinline__ float GroupBroadcast(float v)
-{
-    const uint32_t u = __float_as_uint(v);
-    const auto p = __builtin_amdgcn_permlane16_swap(u, u, false, false);  // {g0 g0 g2 g2}, {g1 g1 g3 g3}
-    const uint32_t s = (g & 1) ? p[1] : p[0];
-    const auto q = __builtin_amdgcn_permlane32_swap(s, s, false, false);
-    return __uint_as_float((g & 2) ? q[1] : q[0]);
 }
 
 // Makes LDS writes of the WAVES waves that work together visible to them.
@@ -183,7 +173,7 @@ __device__ __forceinline__ bool DiagSteps(float (&y)[4], const float (*d)[kT + 4
             }
             y[e] = grp == g ? v : y[e];
         }
-        const float xk = GroupBroadcast<g>(v);
+        const float xk = dev::GroupBroadcast<g>(v);
         // rows past the order come last in a forward solve; in a backward one their steps change nothing
         const bool live = LOWER || k < rows;
         dev::StaticFor<0, 4>([&](auto jc) {

@@ -9,12 +9,13 @@
 // MI355X design: one blocked algorithm for every side / uplo / trans case.
 // op(A) is walked in 128 x 128 diagonal blocks in the order its triangle
 // dictates (forward when the effective factor is lower, backward otherwise):
-//   1. the diagonal block is solved against all right-hand sides by
-//      TrsmDiagKernel: the block goes to LDS (diagonal taken as 1 for a unit
-//      triangle), each lane owns one column (left side) or one row (right
-//      side) of the block of B and runs the substitution in the operation
-//      order of netlib strsm.f, so an order up to 128 (one block) rounds
-//      exactly as the reference's golden;
+//   1. the diagonal block is solved against all right-hand sides in the
+//      operation order of netlib strsm.f, so an order up to 128 (one block)
+//      rounds exactly as the reference's golden: column sweeps on 16 x 16
+//      tiles (TrsmSweepKernel), or, where strsm.f accumulates ascending inner
+//      products, one lane per vector (TrsmInnerKernel).  With several blocks
+//      the updates between them round in the GEMM's order anyway, and the
+//      sweep, whose steps run in parallel over the rows, takes every block;
 //   2. the rest of B is updated by the library's FP32 MFMA GEMM
 //      (aclblasSgemm, alpha -1, beta 1; operands addressed in place in A and
 //      B, transposition through the GEMM's op flags).
@@ -24,12 +25,16 @@
 #include "cann_ops_blas.h"
 #include "device_common.h"
 #include "internal.h"
+#include "tile16.h"
 
 namespace aclblas {
 namespace {
 
 constexpr int kTb = 128;         // diagonal block order
-constexpr int kDiagThreads = 64;  // right-hand-side vectors per workgroup
+constexpr int kVec = 16;         // tile order, and vectors per workgroup of the sweep kernel
+constexpr int kSweepThreads = kTb / kVec * 64;  // one wave per tile of the block
+constexpr int kBlockLoads = kTb * kTb / kSweepThreads;
+constexpr int kDiagThreads = 64;  // vectors per workgroup of the inner-product kernel
 
 // B[i + j ldb] *= alpha (or = 0 when zero), i < m, j < n.
 __global__ __launch_bounds__(256) void TrsmScaleKernel(float* __restrict__ B, int m, int n, int ldb, float alpha,
@@ -45,101 +50,258 @@ __global__ __launch_bounds__(256) void TrsmScaleKernel(float* __restrict__ B, in
     }
 }
 
-// Solves one diagonal block M y = b for `vectors` right-hand-side vectors.  M
+// One diagonal block M y = b for `vectors` right-hand-side vectors.  M
 // (kb x kb) is the block of op(A) for the left side and of op(A)^T for the
 // right side: M(i, j) = A(k0 + i, k0 + j) when readDirect, else
 // A(k0 + j, k0 + i); lower (forward) or upper.  Left side: vector = column c
 // of B, b_i = B(k0 + i, c); right side: vector = row r, b_i = B(r, k0 + i).
-// The substitution follows netlib strsm.f operation for operation: forward
-// and descending-backward as column sweeps (each finished y_k subtracted
-// from the rows still open), ascending-backward (asc) as inner products
-// accumulated from index i + 1 upward; every multiply-subtract rounded
-// separately; the diagonal divides (left) or multiplies by its reciprocal
-// (right); a unit diagonal is not read.  One lane per vector, the vectors'
-// values in LDS columns (conflict-free), the block in LDS.
-template <bool LEFT>
-__global__ __launch_bounds__(kDiagThreads) void TrsmDiagKernel(const float* __restrict__ A, int lda,
-                                                             float* __restrict__ B, int ldb, int k0, int kb,
-                                                             int vectors, int readDirect, int unit, int lowerM,
-                                                             int asc)
+// The substitution follows netlib strsm.f operation for operation: every
+// multiply-subtract rounded separately (so no matrix instruction), the
+// diagonal divides (left) or multiplies by its reciprocal (right), a unit
+// diagonal is not read.
+struct DiagArgs {
+    const float* A;
+    float* B;
+    int lda, ldb;
+    int k0, kb;
+    int vectors;
+    int readDirect, unit;
+};
+
+__device__ __forceinline__ float LoadM(const DiagArgs& p, int i, int j)
 {
-    __shared__ float T[kTb][kTb + 1];
+    return p.readDirect != 0 ? dev::G(p.A)[(p.k0 + i) + static_cast<size_t>(p.k0 + j) * p.lda]
+                             : dev::G(p.A)[(p.k0 + j) + static_cast<size_t>(p.k0 + i) * p.lda];
+}
+
+template <bool LEFT>
+__device__ __forceinline__ size_t BOffset(const DiagArgs& p, int i, int vec)
+{
+    return LEFT ? (p.k0 + i) + static_cast<size_t>(vec) * p.ldb : vec + static_cast<size_t>(p.k0 + i) * p.ldb;
+}
+
+// Column sweeps (forward: k ascending, else descending; each finished y_k is
+// subtracted from the rows still open), 16 vectors per workgroup of eight
+// waves.  Wave I holds rows 16 I .. 16 I + 15 as one tile (dev::F32x4 layout);
+// in phase J wave J solves its 16 x 16 block and publishes y, then the waves
+// behind it subtract the block's 16 columns in k order, wave J + 1 first of
+// all finishing its tile.  The block lies in LDS as [column][row], so a wave
+// reads the four rows of a lane at once.
+//
+// What bounds it: the chain of kb quotients, broadcasts and subtractions.  One
+// lane per vector with its values in LDS (before) took 255 us for a block of
+// 128 and 1000 vectors: 16 waves on the GPU, one dependent LDS round trip per
+// multiply-subtract; this takes 19 us (504 waves).
+template <bool LEFT, bool FORWARD>
+__global__ __launch_bounds__(kSweepThreads) void TrsmSweepKernel(DiagArgs p)
+{
+    __shared__ __attribute__((aligned(16))) float T[kTb][kTb + 4];  // [column][row]
+    __shared__ float ys[2][kVec][kVec];                             // y of the solved block, [k][vector]
+    const int tid = threadIdx.x;
+    const int lane = dev::LaneId();
+    const int wave = dev::Uniform(tid / dev::kWave);
+    const int r16 = lane & 15;
+    const int grp = lane >> 4;
+    const int nt = (p.kb + kVec - 1) / kVec;
+    const int vec = static_cast<int>(blockIdx.x) * kVec + r16;
+    float x[4];
+    dev::StaticFor<0, 4>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        const int i = kVec * wave + 4 * grp + j;
+        x[j] = dev::G(p.B)[BOffset<LEFT>(p, min(i, p.kb - 1), min(vec, p.vectors - 1))];
+    });
+    // the whole block in flight: unconditional loads at clamped indices (a load
+    // under a lane's condition would be waited for on its own), selected after.
+    // Rows and columns past kb are the identity's: their y is b = 0.
+    float m[kBlockLoads];
+    dev::StaticFor<0, kBlockLoads>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        const int fast = min(tid % kTb, p.kb - 1);
+        const int slow = min(tid / kTb + q * (kSweepThreads / kTb), p.kb - 1);
+        m[q] = p.readDirect != 0 ? LoadM(p, fast, slow) : LoadM(p, slow, fast);
+    });
+    dev::StaticFor<0, 4>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        x[j] = kVec * wave + 4 * grp + j < p.kb && vec < p.vectors ? x[j] : 0.0f;
+    });
+    dev::StaticFor<0, kBlockLoads>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        const int fast = tid % kTb;
+        const int slow = tid / kTb + q * (kSweepThreads / kTb);
+        const int i = p.readDirect != 0 ? fast : slow;
+        const int j = p.readDirect != 0 ? slow : fast;
+        const bool in = i < p.kb && j < p.kb && (i == j ? p.unit == 0 : (FORWARD ? i > j : i < j));
+        T[j][i] = in ? m[q] : (i == j ? 1.0f : 0.0f);
+    });
+    __syncthreads();
+    for (int ph = 0; ph < nt; ++ph) {
+        const int J = FORWARD ? ph : nt - 1 - ph;
+        float (*yb)[kVec] = ys[ph & 1];
+        if (wave == J) {
+            float u[4];
+            dev::StaticFor<0, 4>([&](auto jc) {
+                constexpr int j = decltype(jc)::value;
+                const int i = kVec * J + 4 * grp + j;
+                u[j] = LEFT ? T[i][i] : 1.0f / T[i][i];
+            });
+            dev::StaticFor<0, kVec>([&](auto sc) {
+                constexpr int k = FORWARD ? decltype(sc)::value : kVec - 1 - decltype(sc)::value;
+                constexpr int g = k / 4;
+                constexpr int e = k % 4;
+                const dev::F32x4 d = *reinterpret_cast<const dev::F32x4*>(&T[kVec * J + k][kVec * J + 4 * grp]);
+                const float q = LEFT ? x[e] / u[e] : u[e] * x[e];  // group g holds row k
+                x[e] = grp == g ? q : x[e];
+                const float yk = dev::GroupBroadcast<g>(q);
+                dev::StaticFor<0, 4>([&](auto jc) {
+                    constexpr int j = decltype(jc)::value;
+                    const bool open = FORWARD ? (j > e ? grp >= g : grp > g) : (j < e ? grp <= g : grp < g);
+                    const float z = x[j] - d[j] * yk;
+                    x[j] = open ? z : x[j];
+                });
+            });
+            dev::StaticFor<0, 4>([&](auto jc) {
+                constexpr int j = decltype(jc)::value;
+                yb[4 * grp + j][r16] = x[j];
+            });
+        }
+        __syncthreads();
+        if (FORWARD ? wave > J && wave < nt : wave < J) {
+            dev::StaticFor<0, kVec>([&](auto sc) {
+                constexpr int k = FORWARD ? decltype(sc)::value : kVec - 1 - decltype(sc)::value;
+                const dev::F32x4 d = *reinterpret_cast<const dev::F32x4*>(&T[kVec * J + k][kVec * wave + 4 * grp]);
+                const float yk = yb[k][r16];
+                dev::StaticFor<0, 4>([&](auto jc) {
+                    constexpr int j = decltype(jc)::value;
+                    x[j] = x[j] - d[j] * yk;
+                });
+            });
+        }
+    }
+    dev::StaticFor<0, 4>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        const int i = kVec * wave + 4 * grp + j;
+        if (i < p.kb && vec < p.vectors) {
+            dev::G(p.B)[BOffset<LEFT>(p, i, vec)] = x[j];
+        }
+    });
+}
+
+// Ascending inner products, the order strsm.f uses for the backward solves
+// with A itself on the right or A^T on the left: y_i takes the products with
+// y_{i+1}, y_{i+2}, ... in that order, so each y_i starts with the value
+// solved last and the whole block is one chain of kb^2 / 2 subtractions: one
+// lane per vector, the vectors' values in LDS columns.  128 x 1000: 210 us
+// with an LDS round trip per product, 159 us.
+template <bool LEFT>
+__global__ __launch_bounds__(kDiagThreads) void TrsmInnerKernel(DiagArgs p)
+{
+    __shared__ __attribute__((aligned(16))) float T[kTb][kTb];  // [row][column]
     __shared__ float ys[kTb][kDiagThreads];
     const int tid = threadIdx.x;
-    for (int e = tid; e < kb * kb; e += kDiagThreads) {
-        const int i = e % kb;
-        const int j = e / kb;
-        float v = 0.0f;
-        if (i == j) {
-            v = unit == 0 ? A[(k0 + i) + static_cast<size_t>(k0 + i) * lda] : 1.0f;
-        } else if (lowerM != 0 ? i > j : i < j) {
-            v = readDirect != 0 ? A[(k0 + i) + static_cast<size_t>(k0 + j) * lda]
-                                : A[(k0 + j) + static_cast<size_t>(k0 + i) * lda];
+#pragma unroll 8
+    for (int i = 0; i < p.kb; ++i) {
+        float m[kTb / kDiagThreads];
+#pragma unroll
+        for (int q = 0; q < kTb / kDiagThreads; ++q) {
+            m[q] = LoadM(p, i, min(tid + q * kDiagThreads, p.kb - 1));
         }
-        T[i][j] = v;
+#pragma unroll
+        for (int q = 0; q < kTb / kDiagThreads; ++q) {
+            const int j = tid + q * kDiagThreads;
+            T[i][j] = j < p.kb && (i == j ? p.unit == 0 : i < j) ? m[q] : (i == j ? 1.0f : 0.0f);
+        }
     }
-    const int vec = blockIdx.x * kDiagThreads + tid;
-    const bool valid = vec < vectors;
-    for (int i = 0; i < kb; ++i) {
-        ys[i][tid] = !valid ? 0.0f
-                            : (LEFT ? B[(k0 + i) + static_cast<size_t>(vec) * ldb]
-                                    : B[vec + static_cast<size_t>(k0 + i) * ldb]);
+    const int vec = static_cast<int>(blockIdx.x) * kDiagThreads + tid;
+    const bool valid = vec < p.vectors;
+#pragma unroll 8
+    for (int i = 0; i < p.kb; ++i) {
+        const float v = dev::G(p.B)[BOffset<LEFT>(p, i, min(vec, p.vectors - 1))];
+        ys[i][tid] = valid ? v : 0.0f;
+    }
+    for (int i = p.kb; i < kTb; ++i) {
+        ys[i][tid] = 0.0f;  // columns past kb: zero products
     }
     __syncthreads();
-    auto diag = [&](float y, int k) -> float {
-        if (LEFT) {
-            return y / T[k][k];
-        }
-        const float r = 1.0f / T[k][k];
-        return r * y;
+    // eight products at a time, the next eight operands loaded before the
+    // subtractions that use these
+    struct Group {
+        dev::F32x4 m[2];
+        float y[8];
     };
-    if (lowerM != 0) {
-        for (int k = 0; k < kb; ++k) {
-            const float yk = diag(ys[k][tid], k);
-            ys[k][tid] = yk;
-            for (int i = k + 1; i < kb; ++i) {
-                ys[i][tid] = ys[i][tid] - T[i][k] * yk;
+    const auto load = [&](int i, int k) {
+        Group q;
+        q.m[0] = *reinterpret_cast<const dev::F32x4*>(&T[i][k]);
+        q.m[1] = *reinterpret_cast<const dev::F32x4*>(&T[i][k + 4]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            q.y[e] = ys[k + e][tid];
+        }
+        return q;
+    };
+    for (int i = p.kb - 1; i >= 0; --i) {
+        float t = ys[i][tid];
+        const int k0 = (i + 1) & ~7;
+        if (k0 < p.kb) {
+            Group cur = load(i, k0);
+            float prod[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                // entries up to the diagonal: t - (+0) is t
+                prod[e] = k0 + e > i ? cur.m[e / 4][e % 4] * cur.y[e] : 0.0f;
+            }
+            for (int k = k0 + 8; k < p.kb; k += 8) {
+                cur = load(i, k);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    t = t - prod[e];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    prod[e] = cur.m[e / 4][e % 4] * cur.y[e];
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                t = t - prod[e];
             }
         }
-    } else if (asc != 0) {
-        for (int i = kb - 1; i >= 0; --i) {
-            float t = ys[i][tid];
-            for (int k = i + 1; k < kb; ++k) {
-                t = t - T[i][k] * ys[k][tid];
-            }
-            ys[i][tid] = diag(t, i);
-        }
-    } else {
-        for (int k = kb - 1; k >= 0; --k) {
-            const float yk = diag(ys[k][tid], k);
-            ys[k][tid] = yk;
-            for (int i = 0; i < k; ++i) {
-                ys[i][tid] = ys[i][tid] - T[i][k] * yk;
-            }
-        }
+        ys[i][tid] = LEFT ? t / T[i][i] : (1.0f / T[i][i]) * t;
     }
     if (valid) {
-        for (int i = 0; i < kb; ++i) {
-            if (LEFT) {
-                B[(k0 + i) + static_cast<size_t>(vec) * ldb] = ys[i][tid];
-            } else {
-                B[vec + static_cast<size_t>(k0 + i) * ldb] = ys[i][tid];
-            }
+        for (int i = 0; i < p.kb; ++i) {
+            dev::G(p.B)[BOffset<LEFT>(p, i, vec)] = ys[i][tid];
         }
     }
 }
 
-void LaunchDiag(hipStream_t st, bool left, const float* A, int lda, float* B, int ldb, int k0, int kb, int vectors,
-                int readDirect, int unit, int lowerM, int asc)
+// inner: ascending inner products instead of the backward column sweep.
+void LaunchDiag(hipStream_t st, bool left, const DiagArgs& p, bool forward, bool inner)
 {
-    const dim3 grid(static_cast<unsigned>((vectors + kDiagThreads - 1) / kDiagThreads));
-    const dim3 block(kDiagThreads);
+    if (inner) {
+        const dim3 grid(static_cast<unsigned>((p.vectors + kDiagThreads - 1) / kDiagThreads));
+        if (left) {
+            hipLaunchKernelGGL(TrsmInnerKernel<true>, grid, dim3(kDiagThreads), 0, st, p);
+        } else {
+            hipLaunchKernelGGL(TrsmInnerKernel<false>, grid, dim3(kDiagThreads), 0, st, p);
+        }
+        return;
+    }
+    const dim3 grid(static_cast<unsigned>((p.vectors + kVec - 1) / kVec));
+    const dim3 block(kSweepThreads);
     if (left) {
-        hipLaunchKernelGGL(TrsmDiagKernel<true>, grid, block, 0, st, A, lda, B, ldb, k0, kb, vectors, readDirect, unit,
-                           lowerM, asc);
+        if (forward) {
+            hipLaunchKernelGGL((TrsmSweepKernel<true, true>), grid, block, 0, st, p);
+        } else {
+            hipLaunchKernelGGL((TrsmSweepKernel<true, false>), grid, block, 0, st, p);
+        }
     } else {
-        hipLaunchKernelGGL(TrsmDiagKernel<false>, grid, block, 0, st, A, lda, B, ldb, k0, kb, vectors, readDirect,
-                           unit, lowerM, asc);
+        if (forward) {
+            hipLaunchKernelGGL((TrsmSweepKernel<false, true>), grid, block, 0, st, p);
+        } else {
+            hipLaunchKernelGGL((TrsmSweepKernel<false, false>), grid, block, 0, st, p);
+        }
     }
 }
 
@@ -211,17 +373,17 @@ extern "C" aclblasStatus_t aclblasStrsm(aclblasHandle_t handle, aclblasSideMode_
     const bool forward = left ? opLower : !opLower;
     // M(i, j) read directly from A when M is A itself: left N, right T.
     const int readDirect = (left != tr) ? 1 : 0;
-    // backward solves whose strsm.f loop accumulates inner products upward
-    const int asc = (!forward && left == tr) ? 1 : 0;
     const int vectors = left ? n : m;
     const int blocks = (k + kTb - 1) / kTb;
+    // backward solves whose strsm.f loop accumulates inner products upward
+    const bool inner = !forward && left == tr && blocks == 1;
     const float minus1 = -1.0f;
     const float one = 1.0f;
     for (int s = 0; s < blocks; ++s) {
         const int bi = forward ? s : blocks - 1 - s;
         const int k0 = bi * kTb;
         const int kb = k - k0 < kTb ? k - k0 : kTb;
-        LaunchDiag(st, left, A, lda, B, ldb, k0, kb, vectors, readDirect, unit, forward ? 1 : 0, asc);
+        LaunchDiag(st, left, DiagArgs{A, B, lda, ldb, k0, kb, vectors, readDirect, unit}, forward, inner);
         aclblasStatus_t rs = LaunchStatus("aclblasStrsm");
         if (rs != ACLBLAS_STATUS_SUCCESS) {
             return rs;

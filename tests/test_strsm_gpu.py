@@ -175,3 +175,20 @@ def test_strsm_graph_capture(handle):
     finally:
         torch.cuda.synchronize()
         h.destroy()
+
+
+@pytest.mark.parametrize("dim", [1, 15, 16, 17, 100, 127, 128])
+@pytest.mark.parametrize("side", ["LEFT", "RIGHT"])
+@pytest.mark.parametrize("uplo", ["LOWER", "UPPER"])
+@pytest.mark.parametrize("trans", ["N", "T"])
+@pytest.mark.parametrize("diag", ["NON_UNIT", "UNIT"])
+def test_strsm_one_block_bitwise(handle, dim, side, uplo, trans, diag):
+    """Orders of one diagonal block (at the edges of its 16-row tiles) round exactly as the oracle's netlib order."""
+    m, n = (dim, 37) if side == "LEFT" else (37, dim)
+    row = {"side": side, "uplo": uplo, "trans": trans, "diag": diag, "m": str(m), "n": str(n),
+           "lda": str(dim + 1), "ldb": str(m + 2), "alpha": "1.0", "a": "RANDOM_NORM", "b": "RANDOM_NORM",
+           "random_seed": str(dim)}
+    a, b = _inputs(row)
+    st, out = _call(handle, row, a, b)
+    assert st == 0
+    assert np.array_equal(out[:(m + 2) * n], _gold(row, a, b)[:(m + 2) * n])

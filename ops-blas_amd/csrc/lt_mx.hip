@@ -19,33 +19,52 @@
 // and the rounding to D's type are fused in the epilogue, and D is written
 // once.
 //
-// One workgroup of four waves per 64 x 64 tile of D, each wave 32 x 32 (two
-// by two MFMA tiles); K advances 128 elements per step through LDS, where
-// every operand is held K-contiguous per row (a row of A or a column of B),
-// 128 bytes (FP8) or 64 bytes (FP4, two elements per byte, low nibble first)
-// per step, plus four scale bytes per row.  Operands stored K-contiguous are
-// copied 16 bytes at a time; the others are transposed on the way into LDS.
-// Rows or columns past m / n, and K blocks past k (k is a multiple of 32)
-// read as zeros with scale 1.  A scale byte of 0 makes its block contribute
-// 0, the reference golden's decoding of E8M0 0 (the instruction would scale
-// by 2^-127).
+// One workgroup of four waves (2 x 2) per BT x BT tile of D (eight, 2 x 4, for
+// 256 x 256); K advances 128 elements per stage, one barrier per stage.  Aligned
+// operands go straight to a ring of LDS stages (LtMxDmaKernel); others through
+// registers into two LDS buffers, the next stage's loads in flight while the
+// matrix instructions consume this one (LtMxKernel).  An operand stored K-contiguous keeps its rows in LDS (128 bytes for
+// FP8, 64 for FP4) and is read 16 bytes at a time; one stored the other way
+// keeps its K rows and is read with the transposing ds_read_b64_tr_b8 / _b4, so
+// nothing is transposed on the way in.  16-byte chunks are XOR-swizzled so that
+// both reads are free of bank conflicts.  Loads are 16 bytes at any alignment;
+// only chunks that would end past the operand are read byte by byte.  Rows or
+// columns past m / n read other (valid) elements whose results are not stored;
+// K blocks past k (k is a multiple of 32) read as zeros with scale 1.  A scale
+// byte of 0 makes its block contribute 0, the reference golden's decoding of
+// E8M0 0 (the instruction would scale by 2^-127): a stage whose scales hold a
+// zero byte has those blocks' data zeroed in LDS.
+//
+// What bounds it: the LDS round trips at the start of a stage (its fragments
+// can only be read after the barrier) against 32 matrix instructions per wave
+// with 256 x 256 tiles and 16 with 128 x 128; the larger tile, whose two waves
+// per SIMD also cover for each other, reaches 1.4 PFLOP/s.  4096^3, BF16 out, A
+// and B K-contiguous (NT) / both row-contiguous (TN): MXFP8 332 -> 84 / 2490
+// -> 88 us, MXFP4 191 -> 76 / 1523 -> 62 us (before: 64 x 64 tiles, element-wise
+// transposes, no load in flight during the products).  Fragments of the next
+// stage held in registers during the products were slower (174 us: the
+// compiler moves them through the accumulation registers).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
 
+#include "device_common.h"
 #include "drivers.h"
 #include "internal.h"
+#include "lds_dma.h"
 
 namespace aclblas {
 namespace {
 
-constexpr int kTile = 64;
-constexpr int kThreads = 256;
-constexpr int kStepK = 128;     // K elements per step (one MFMA per fragment pair)
-constexpr int kPad = 16;        // bytes of padding per LDS row
+constexpr int kStepK = 128;     // K elements per stage (one MFMA per fragment pair)
 
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4Any __attribute__((aligned(1)));
+typedef uint16_t u16Any __attribute__((aligned(1)));
+typedef int V2i32 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) V2i32 LdsV2i32;
 
 struct MxArgs {
     const uint8_t* A;
@@ -58,94 +77,256 @@ struct MxArgs {
     long long pitchB;
     int m, n, k;
     int ldc, ldd;
-    int transA, transB; // 0 = N
-    int vecA, vecB;     // 16-byte copies possible (aligned base and pitch)
+    int tilesM, tilesN;
+    int vecC, vecD;     // four consecutive elements of a row can move as one vector
+    int bf16Out;
+    int dma;            // the direct-to-LDS kernel may run
     float alpha, beta;
 };
 
-// Scale byte of row `row` (of A: m index; of B: n index) and K block b.
-// kMajorPairs: the [b / 2][rows][2] layout, else [rows][2 ceil(k / 64)].
-__device__ __forceinline__ uint8_t ScaleAt(const uint8_t* s, bool kMajorPairs, int rows, int k, int row, int b)
-{
-    if (kMajorPairs) {
-        return s[static_cast<size_t>(b >> 1) * 2 * rows + 2 * row + (b & 1)];
-    }
-    const int stride = ((k + 63) / 64) * 2;
-    return s[static_cast<size_t>(row) * stride + b];
-}
+// Workgroup of a BT x BT tile: 2 x 2 waves, or 2 x 4 for the largest tile.
+constexpr int Threads(int bt) { return bt == 256 ? 512 : 256; }
+constexpr int WavesN(int bt) { return bt == 256 ? 4 : 2; }
 
-// Loads one operand's 64-row step into LDS rows of `rowBytes` data bytes.
-// kContig: element (row, kk) of the operand is stored at row * pitch + kk
-// (bytes kk / 2 for FP4), else at kk * pitch + row.
-template <bool FP4>
-__device__ __forceinline__ void LoadOperand(uint8_t* lds, uint8_t* sc, const uint8_t* X, long long pitch,
-                                            bool kContig, bool vec, int row0, int rows, int k0, int k,
-                                            const uint8_t* scale, bool kMajorPairs)
-{
-    constexpr int kRowBytes = FP4 ? kStepK / 2 : kStepK;
-    constexpr int kLd = kRowBytes + kPad;
-    const int t = threadIdx.x;
-    const int kBytes0 = FP4 ? k0 / 2 : k0;       // byte offset of this step along K (K-contiguous storage)
-    const int kBytesEnd = FP4 ? k / 2 : k;
-    if (kContig) {
-        // 16-byte chunks: kRowBytes / 16 per row
-        constexpr int kChunks = kRowBytes / 16;
-        for (int e = t; e < kTile * kChunks; e += kThreads) {
-            const int r = e / kChunks;
-            const int c = e % kChunks;
-            const int row = row0 + r;
-            const int kb = kBytes0 + 16 * c;
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (row < rows && kb < kBytesEnd) {
-                const uint8_t* src = X + static_cast<size_t>(row) * pitch + kb;
-                if (vec) {
-                    v = *reinterpret_cast<const uint4*>(src);
+// One operand's tile of BT rows (m or n indices).  KC: stored K-contiguous
+// (element (row, kk) at row * pitch + kk, FP4 nibbles two per byte), else
+// row-contiguous (at kk * pitch + row).
+template <bool FP4, bool KC, int BT>
+struct Operand {
+    static constexpr int kThreads = Threads(BT);
+    static constexpr int kRowBytes = KC ? (FP4 ? 64 : 128) : (FP4 ? BT / 2 : BT);  // an LDS row
+    static constexpr int kRowChunks = kRowBytes / 16;
+    static constexpr int kBytes = BT * (FP4 ? 64 : 128);                           // a stage
+    static constexpr int kLoads = kBytes / 16 / kThreads;
+    const uint8_t* src[kLoads];  // this thread's chunks at stage 0
+    const uint8_t* end;          // past the operand's last byte
+    long long step;
+    int kEnd;                    // K elements
+    bool inside;                 // row-contiguous: every chunk of the tile inside its row
+
+    // swizzle key of LDS row r: rows that are read together land in distinct
+    // chunks of a 256-byte window
+    __device__ __forceinline__ static int Key(int r)
+    {
+        if (KC) {
+            return FP4 ? (r >> 1) & 3 : r & 7;
+        }
+        return kRowChunks >= 8 ? r & 7 : (kRowChunks == 4 ? (r >> 2) & 3 : (r >> 3) & 1);
+    }
+    __device__ __forceinline__ static uint32_t Offset(int r, int chunk)
+    {
+        return static_cast<uint32_t>(r * kRowBytes + ((chunk ^ Key(r)) << 4));
+    }
+
+    __device__ __forceinline__ void Setup(const uint8_t* X, long long pitch, int row0, int rows, int k)
+    {
+        const int t = threadIdx.x;
+        const int rowBytes = FP4 ? (rows + 1) / 2 : rows;  // row-contiguous storage
+        const int byte0 = FP4 ? row0 / 2 : row0;
+#pragma unroll
+        for (int q = 0; q < kLoads; ++q) {
+            const int id = t + kThreads * q;
+            const int r = id / kRowChunks;
+            const int c = id % kRowChunks;
+            src[q] = KC ? X + static_cast<long long>(min(row0 + r, rows - 1)) * pitch + 16 * c
+                        : X + static_cast<long long>(r) * pitch + byte0 + 16 * c;
+        }
+        step = KC ? static_cast<long long>(kRowBytes) : kStepK * pitch;
+        end = KC ? nullptr : X + static_cast<long long>(k - 1) * pitch + rowBytes;
+        kEnd = k;
+        inside = KC || byte0 + kRowBytes <= rowBytes;
+    }
+
+    __device__ __forceinline__ void Load(int stage, u32x4 (&v)[kLoads]) const
+    {
+        const long long off = stage * step;
+        const int left = kEnd - stage * kStepK;  // K elements from this stage on
+        if (left >= kStepK && inside) {
+#pragma unroll
+            for (int q = 0; q < kLoads; ++q) {
+                v[q] = *(const ACL_GLOBAL u32x4Any*)(src[q] + off);
+            }
+            return;
+        }
+        const int t = threadIdx.x;
+#pragma unroll
+        for (int q = 0; q < kLoads; ++q) {
+            const int id = t + kThreads * q;
+            const uint8_t* p = src[q] + off;
+            u32x4 w = {0u, 0u, 0u, 0u};
+            if (KC) {
+                if ((id % kRowChunks) * (FP4 ? 32 : 16) < left) {
+                    w = *(const ACL_GLOBAL u32x4Any*)p;
+                }
+            } else if (id / kRowChunks < left) {
+                if (p + 16 <= end) {
+                    w = *(const ACL_GLOBAL u32x4Any*)p;
                 } else {
-                    uint32_t w[4];
-                    for (int i = 0; i < 4; ++i) {
-                        w[i] = static_cast<uint32_t>(src[4 * i]) | (static_cast<uint32_t>(src[4 * i + 1]) << 8) |
-                               (static_cast<uint32_t>(src[4 * i + 2]) << 16) |
-                               (static_cast<uint32_t>(src[4 * i + 3]) << 24);
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        if (p + i < end) {
+                            w[i / 4] |= static_cast<uint32_t>(dev::LoadG<uint8_t>(p + i)) << (8 * (i % 4));
+                        }
                     }
-                    v = make_uint4(w[0], w[1], w[2], w[3]);
                 }
             }
-            *reinterpret_cast<uint4*>(lds + r * kLd + 16 * c) = v;
+            v[q] = w;
         }
-    } else if constexpr (!FP4) {
-        // element (row, kk) at kk * pitch + row: one byte per (row, kk)
-        for (int e = t; e < kTile * kStepK; e += kThreads) {
-            const int r = e % kTile;
-            const int kk = e / kTile;
-            const int row = row0 + r;
-            const int kg = k0 + kk;
-            lds[r * kLd + kk] = (row < rows && kg < k) ? X[static_cast<size_t>(kg) * pitch + row] : 0;
+    }
+
+    // The sources of a direct-to-LDS stage: a wave instruction fills 64
+    // consecutive 16-byte slots, so each lane fetches the chunk that belongs in
+    // its slot.  Rows past the edge, and chunks past a row's end (row-contiguous
+    // rows are whole chunks then), read clamped addresses.
+    __device__ __forceinline__ void SetupDma(const uint8_t* X, long long pitch, int row0, int rows)
+    {
+        const int t = threadIdx.x;
+        const int rowBytes = FP4 ? rows / 2 : rows;
+        const int byte0 = FP4 ? row0 / 2 : row0;
+#pragma unroll
+        for (int q = 0; q < kLoads; ++q) {
+            const int id = t + kThreads * q;
+            const int r = id / kRowChunks;
+            const int c = (id % kRowChunks) ^ Key(r);
+            src[q] = KC ? X + static_cast<long long>(min(row0 + r, rows - 1)) * pitch + 16 * c
+                        : X + static_cast<long long>(r) * pitch + min(byte0 + 16 * c, rowBytes - 16);
         }
-    } else {
-        // FP4: nibble (row, kk) at byte kk * pitch + row / 2, low nibble for even rows; an LDS byte packs
-        // K elements 2q (low) and 2q + 1 (high) of one row
-        for (int e = t; e < kTile * (kStepK / 2); e += kThreads) {
-            const int r = e % kTile;
-            const int q = e / kTile;
-            const int row = row0 + r;
-            const int kg = k0 + 2 * q;
-            uint8_t out = 0;
-            if (row < rows && kg < k) {
-                const uint8_t lo = X[static_cast<size_t>(kg) * pitch + row / 2];
-                const uint8_t hi = X[static_cast<size_t>(kg + 1) * pitch + row / 2];
-                const int sh = (row & 1) * 4;
-                out = static_cast<uint8_t>(((lo >> sh) & 0xF) | (((hi >> sh) & 0xF) << 4));
+        step = KC ? static_cast<long long>(kRowBytes) : kStepK * pitch;
+    }
+    __device__ __forceinline__ void Issue(int stage, uint8_t* lds, int wave) const
+    {
+        const uint32_t base = dev::LdsAddr(lds);
+#pragma unroll
+        for (int q = 0; q < kLoads; ++q) {
+            dev::LdsDma16(src[q] + stage * step,
+                          __builtin_amdgcn_readfirstlane(base + 1024u * (wave + kThreads / 64 * q)));
+        }
+    }
+
+    __device__ __forceinline__ void Store(uint8_t* lds, const u32x4 (&v)[kLoads]) const
+    {
+        const int t = threadIdx.x;
+#pragma unroll
+        for (int q = 0; q < kLoads; ++q) {
+            const int id = t + kThreads * q;
+            *reinterpret_cast<u32x4*>(lds + Offset(id / kRowChunks, id % kRowChunks)) = v[q];
+        }
+    }
+
+    // A lane's operand of v_mfma_scale_f32_16x16x128_f8f6f4 for the 16 rows from
+    // row0 of the tile (row0 a multiple of 16).  The instruction's K slots,
+    // established on the GPU, are:
+    //   FP8: the lane's bytes 0-15 are slots 16 g .. 16 g + 15 and bytes 16-31
+    //        are slots 64 + 16 g .. 64 + 16 g + 15 (g = lane / 16); the scale the
+    //        lane supplies covers slots 32 g .. 32 g + 31;
+    //   FP4: the lane's 32 elements are slots 32 g .. 32 g + 31 and its scale
+    //        covers them.
+    // Slot s holds K element k0 + s.  ds_read_b64_tr_b8: in a group of 16 lanes,
+    // lane 2 e + a pointing at rows 8a .. 8a + 7 of K element e gives lane i row
+    // i, elements 0..7; ds_read_b64_tr_b4: lane e pointing at the 16 rows of K
+    // element e gives lane i row i, elements 0..15.
+    __device__ __forceinline__ static i32x8 Fragment(const uint8_t* lds, int row0, int lane)
+    {
+        const int g = lane >> 4;
+        const int j = lane & 15;
+        if constexpr (KC) {
+            const int r = row0 + j;
+            const u32x4 lo = *reinterpret_cast<const u32x4*>(lds + Offset(r, g));
+            if constexpr (FP4) {
+                return i32x8{static_cast<int>(lo.x), static_cast<int>(lo.y), static_cast<int>(lo.z),
+                             static_cast<int>(lo.w), 0, 0, 0, 0};
+            } else {
+                const u32x4 hi = *reinterpret_cast<const u32x4*>(lds + Offset(r, 4 + g));
+                return i32x8{static_cast<int>(lo.x), static_cast<int>(lo.y), static_cast<int>(lo.z),
+                             static_cast<int>(lo.w), static_cast<int>(hi.x), static_cast<int>(hi.y),
+                             static_cast<int>(hi.z), static_cast<int>(hi.w)};
             }
-            lds[r * kLd + q] = out;
+        } else if constexpr (FP4) {
+            V2i32 v[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const uint8_t* p = lds + Offset(32 * g + 16 * h + j, row0 >> 5) + ((row0 >> 4) & 1) * 8;
+                v[h] = __builtin_amdgcn_ds_read_tr4_b64_v2i32((LdsV2i32*)p);
+            }
+            return i32x8{v[0].x, v[0].y, v[1].x, v[1].y, 0, 0, 0, 0};
+        } else {
+            V2i32 v[4];
+#pragma unroll
+            for (int h = 0; h < 4; ++h) {
+                const int k = (h >> 1) * 64 + 16 * g + 8 * (h & 1) + (j >> 1);
+                const uint8_t* p = lds + Offset(k, row0 >> 4) + 8 * (j & 1);
+                v[h] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((LdsV2i32*)p);
+            }
+            return i32x8{v[0].x, v[0].y, v[1].x, v[1].y, v[2].x, v[2].y, v[3].x, v[3].y};
         }
     }
-    // scales: four K blocks of 32 per step
-    for (int e = t; e < kTile * 4; e += kThreads) {
-        const int r = e / 4;
-        const int b = (k0 / 32) + (e % 4);
-        const int row = row0 + r;
-        sc[e] = (row < rows && 32 * b < k) ? ScaleAt(scale, kMajorPairs, rows, k, row, b) : static_cast<uint8_t>(127);
+};
+
+// Zeroes in LDS the blocks of the wave's rows (row0 .. row0 + ROWS - 1 of the
+// operand's tile, one per lane) whose scale byte is 0; scales(row) gives a
+// row's four.  Other waves that use the rows write the same zeros before they
+// read them, so no barrier is needed; and no accumulator is live across the
+// branch (one would be moved to and from the accumulation registers on every
+// stage).
+template <typename Op, bool FP4, bool KC, int ROWS, typename Scales>
+__device__ __forceinline__ void ZeroBlocks(uint8_t* lds, int row0, int lane, Scales scales)
+{
+    constexpr int kSlabs = ROWS > 64 ? ROWS / 64 : 1;
+    uint32_t s[kSlabs];
+    uint32_t z = 0;
+#pragma unroll
+    for (int q = 0; q < kSlabs; ++q) {
+        s[q] = scales(row0 + 64 * q + lane % min(ROWS, 64));
+        z |= (s[q] - 0x01010101u) & ~s[q] & 0x80808080u;  // 0 exactly when no byte is 0
     }
+    if (__builtin_amdgcn_ballot_w64(z != 0u) == 0) {
+        return;
+    }
+    for (int e = 0; e < 4 * kSlabs; ++e) {
+        const int b = e & 3;
+        const int row = row0 + 64 * (e >> 2) + lane % min(ROWS, 64);
+        if (((s[e >> 2] >> (8 * b)) & 0xFFu) != 0u) {
+            continue;
+        }
+        if constexpr (KC) {
+            constexpr int kChunks = FP4 ? 1 : 2;
+            for (int c = 0; c < kChunks; ++c) {
+                *reinterpret_cast<u32x4*>(lds + Op::Offset(row, kChunks * b + c)) = u32x4{0u, 0u, 0u, 0u};
+            }
+        } else if constexpr (!FP4) {
+            for (int k = 32 * b; k < 32 * b + 32; ++k) {
+                lds[Op::Offset(k, row >> 4) + (row & 15)] = 0;
+            }
+        } else {
+            // the neighbouring row shares the byte
+            for (int k = 32 * b; k < 32 * b + 32; ++k) {
+                const uint32_t at = Op::Offset(k, row >> 5) + ((row & 31) >> 1);
+                atomicAnd(reinterpret_cast<uint32_t*>(lds + (at & ~3u)),
+                          ~(0xFu << (8 * (at & 3u) + 4 * (row & 1))));
+            }
+        }
+    }
+}
+
+// The four scale bytes of a stage (K blocks 4 s .. 4 s + 3) of matrix row `row`
+// (of `rows`), as two pairs.  pairsMajor: the [b / 2][rows][2] layout, else
+// [rows][2 ceil(k / 64)].  Blocks past k scale by 1.
+__device__ __forceinline__ uint32_t LoadScales(const uint8_t* s, bool pairsMajor, int rows, int row, int stage, int k)
+{
+    const int pairs = (k + 63) / 64;
+    uint32_t v = 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int pb = 2 * stage + h;
+        const int at = min(pb, pairs - 1);
+        const long long off = pairsMajor ? (static_cast<long long>(at) * rows + row) * 2
+                                         : (static_cast<long long>(row) * pairs + at) * 2;
+        uint32_t w = *(const ACL_GLOBAL u16Any*)(s + off);
+        w = 64 * pb + 32 < k ? w : ((w & 0xFFu) | 0x7F00u);
+        w = pb < pairs ? w : 0x7F7Fu;
+        v |= w << (16 * h);
+    }
+    return v;
 }
 
 __device__ __forceinline__ uint16_t Bf16Rne(float f)
@@ -158,105 +339,384 @@ __device__ __forceinline__ uint16_t Bf16Rne(float f)
     return static_cast<uint16_t>(u >> 16);
 }
 
-// One lane's operand of v_mfma_scale_f32_16x16x128_f8f6f4 for the step: `row`
-// points at the LDS row (K-contiguous bytes of the step), `sc` at its four
-// block scales, g = lane / 16.  The instruction's K slots, established on the
-// GPU, are:
-//   FP8: the lane's bytes 0-15 are slots 16 g .. 16 g + 15 and bytes 16-31 are
-//        slots 64 + 16 g .. 64 + 16 g + 15; the scale the lane supplies covers
-//        slots 32 g .. 32 g + 31 (held by lane groups 2 (g % 2) .. + 1);
-//   FP4: the lane's 32 elements are slots 32 g .. 32 g + 31 and its scale
-//        covers them.
-// Slot s holds K element k0 + s, so each supplied scale is that of the step's
-// K block g.  A zero scale byte zeroes the data of its block (scale 1 then).
-template <bool FP4>
-__device__ __forceinline__ i32x8 Fragment(const uint8_t* row, const uint8_t* sc, int g, int& scale)
+// One 2-byte value per lane to consecutive LDS dwords (zero-extended); as
+// dev::LdsDma16 otherwise.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void LdsDma2(const void* g, uint32_t lds)
 {
-    const int s = sc[g];
-    scale = s == 0 ? 127 : s;
-    if constexpr (FP4) {
-        const uint4 v = s == 0 ? make_uint4(0, 0, 0, 0) : *reinterpret_cast<const uint4*>(row + 16 * g);
-        return i32x8{static_cast<int>(v.x), static_cast<int>(v.y), static_cast<int>(v.z), static_cast<int>(v.w),
-                     0, 0, 0, 0};
-    } else {
-        // bytes 0-15 belong to block g / 2, bytes 16-31 to block 2 + g / 2
-        const uint4 lo = sc[g >> 1] == 0 ? make_uint4(0, 0, 0, 0) : *reinterpret_cast<const uint4*>(row + 16 * g);
-        const uint4 hi =
-            sc[2 + (g >> 1)] == 0 ? make_uint4(0, 0, 0, 0) : *reinterpret_cast<const uint4*>(row + 64 + 16 * g);
-        return i32x8{static_cast<int>(lo.x), static_cast<int>(lo.y), static_cast<int>(lo.z), static_cast<int>(lo.w),
-                     static_cast<int>(hi.x), static_cast<int>(hi.y), static_cast<int>(hi.z), static_cast<int>(hi.w)};
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_ushort %0, off" : : "v"(g), "s"(lds)
+                 : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
+// The tile a workgroup computes: consecutive tiles on one XCD, walked in
+// groups of eight tile rows that share its L2.
+template <int BT>
+__device__ __forceinline__ void TileOf(const MxArgs& p, int& m0, int& n0)
+{
+    int bid = static_cast<int>(blockIdx.x);
+    if (gridDim.x % 8 == 0) {
+        bid = (bid % 8) * (static_cast<int>(gridDim.x) / 8) + bid / 8;
     }
+    const int perGroup = 8 * p.tilesN;
+    const int firstM = bid / perGroup * 8;
+    const int groupRows = min(8, p.tilesM - firstM);
+    const int inGroup = bid - bid / perGroup * perGroup;
+    m0 = (firstM + inGroup % groupRows) * BT;
+    n0 = inGroup / groupRows * BT;
 }
 
-template <bool FP4, bool BF16OUT>
-__global__ __launch_bounds__(kThreads) void LtMxKernel(MxArgs p)
+// alpha * acc + beta * C for a wave's kF x kF tiles at (mw, nw): the lane holds
+// row r16, columns 4 g + e of each 16 x 16 tile.
+template <int kFA, int kFB>
+__device__ __forceinline__ void StoreTiles(const MxArgs& p, const f32x4 (&acc)[kFA][kFB], int mw, int nw, int lane)
 {
-    constexpr int kRowBytes = FP4 ? kStepK / 2 : kStepK;
-    constexpr int kLd = kRowBytes + kPad;
-    constexpr int kFmt = FP4 ? 4 : 0;  // operand format code: 0 E4M3, 4 E2M1
-    __shared__ __attribute__((aligned(16))) uint8_t sA[kTile * kLd];
-    __shared__ __attribute__((aligned(16))) uint8_t sB[kTile * kLd];
-    __shared__ uint8_t sSA[kTile * 4];
-    __shared__ uint8_t sSB[kTile * 4];
-
-    const int lane = static_cast<int>(threadIdx.x) & 63;
-    const int wave = static_cast<int>(threadIdx.x) >> 6;
-    const int wm = (wave >> 1) * 32;
-    const int wn = (wave & 1) * 32;
     const int r16 = lane & 15;
     const int g = lane >> 4;
-    const int m0 = static_cast<int>(blockIdx.y) * kTile;
-    const int n0 = static_cast<int>(blockIdx.x) * kTile;
-
-    f32x4 acc[2][2];
-    for (int i = 0; i < 2; ++i) {
-        for (int j = 0; j < 2; ++j) {
-            acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        }
-    }
-    // A: row index m, K-contiguous when transA == N; B: row index n, K-contiguous when transB != N.
-    // Scales: A [m][2 ceil(k/64)] when transA == N, else K-major pairs; B the other way round.
-    for (int k0 = 0; k0 < p.k; k0 += kStepK) {
-        LoadOperand<FP4>(sA, sSA, p.A, p.pitchA, p.transA == 0, p.vecA != 0, m0, p.m, k0, p.k, p.scaleA,
-                         p.transA != 0);
-        LoadOperand<FP4>(sB, sSB, p.B, p.pitchB, p.transB != 0, p.vecB != 0, n0, p.n, k0, p.k, p.scaleB,
-                         p.transB == 0);
-        __syncthreads();
-        i32x8 a[2], b[2];
-        int sa[2], sb[2];
-        for (int i = 0; i < 2; ++i) {
-            a[i] = Fragment<FP4>(sA + (wm + 16 * i + r16) * kLd, sSA + (wm + 16 * i + r16) * 4, g, sa[i]);
-        }
-        for (int j = 0; j < 2; ++j) {
-            b[j] = Fragment<FP4>(sB + (wn + 16 * j + r16) * kLd, sSB + (wn + 16 * j + r16) * 4, g, sb[j]);
-        }
-        for (int i = 0; i < 2; ++i) {
-            for (int j = 0; j < 2; ++j) {
-                acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a[i], b[j], acc[i][j], kFmt, kFmt, 0,
-                                                                             sa[i], 0, sb[j]);
+#pragma unroll
+    for (int i = 0; i < kFA; ++i) {
+        const int row = mw + 16 * i + r16;
+#pragma unroll
+        for (int j = 0; j < kFB; ++j) {
+            const int col = nw + 16 * j + 4 * g;
+            if (row >= p.m || col >= p.n) {
+                continue;
             }
-        }
-        __syncthreads();
-    }
-    // epilogue: lane holds rows 4 g + e, column r16 of each 16 x 16 tile
-    for (int i = 0; i < 2; ++i) {
-        for (int j = 0; j < 2; ++j) {
-            const int col = n0 + wn + 16 * j + r16;
+            const int left = min(4, p.n - col);
+            float v[4];
+#pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int row = m0 + wm + 16 * i + 4 * g + e;
-                if (row < p.m && col < p.n) {
-                    float v = p.alpha * acc[i][j][e];
-                    if (p.beta != 0.0f) {
-                        v = fmaf(p.beta, p.C[static_cast<size_t>(row) * p.ldc + col], v);
+                v[e] = p.alpha * acc[i][j][e];
+            }
+            if (p.beta != 0.0f) {
+                const float* c = p.C + static_cast<size_t>(row) * p.ldc + col;
+                if (p.vecC != 0 && left == 4) {
+                    const f32x4 cv = dev::LoadG<f32x4>(c);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        v[e] = fmaf(p.beta, cv[e], v[e]);
                     }
-                    if constexpr (BF16OUT) {
-                        static_cast<uint16_t*>(p.D)[static_cast<size_t>(row) * p.ldd + col] = Bf16Rne(v);
-                    } else {
-                        static_cast<float*>(p.D)[static_cast<size_t>(row) * p.ldd + col] = v;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if (e < left) {
+                            v[e] = fmaf(p.beta, dev::LoadG<float>(c + e), v[e]);
+                        }
+                    }
+                }
+            }
+            const size_t at = static_cast<size_t>(row) * p.ldd + col;
+            if (p.bf16Out != 0) {
+                uint16_t* d = static_cast<uint16_t*>(p.D) + at;
+                const uint32_t lo = Bf16Rne(v[0]) | (static_cast<uint32_t>(Bf16Rne(v[1])) << 16);
+                const uint32_t hi = Bf16Rne(v[2]) | (static_cast<uint32_t>(Bf16Rne(v[3])) << 16);
+                if (p.vecD != 0 && left == 4) {
+                    dev::StoreG(d, make_uint2(lo, hi));
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if (e < left) {
+                            dev::StoreG(d + e, static_cast<uint16_t>((e < 2 ? lo : hi) >> (16 * (e & 1))));
+                        }
+                    }
+                }
+            } else {
+                float* d = static_cast<float*>(p.D) + at;
+                if (p.vecD != 0 && left == 4) {
+                    dev::StoreG(d, f32x4{v[0], v[1], v[2], v[3]});
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if (e < left) {
+                            dev::StoreG(d + e, v[e]);
+                        }
                     }
                 }
             }
         }
+    }
+}
+
+template <bool FP4, bool AK, bool BK, int BT>
+__global__ __launch_bounds__(256, 2) void LtMxKernel(MxArgs p)
+{
+    constexpr int kFmt = FP4 ? 4 : 0;  // operand format code: 0 E4M3, 4 E2M1
+    constexpr int kF = BT / 32;        // 16-row fragments per wave and operand
+    using OpA = Operand<FP4, AK, BT>;
+    using OpB = Operand<FP4, BK, BT>;
+    __shared__ __attribute__((aligned(16))) uint8_t sA[2][OpA::kBytes];
+    __shared__ __attribute__((aligned(16))) uint8_t sB[2][OpB::kBytes];
+    __shared__ uint32_t sS[2][2 * BT];  // scales of A's rows, then of B's
+
+    int m0, n0;
+    TileOf<BT>(p, m0, n0);
+    const int t = static_cast<int>(threadIdx.x);
+    const int lane = t & 63;
+    const int wave = dev::Uniform(t >> 6);
+    const int wm = (wave >> 1) * (BT / 2);
+    const int wn = (wave & 1) * (BT / 2);
+    const int r16 = lane & 15;
+    const int g = lane >> 4;
+
+    OpA oa;
+    OpB ob;
+    oa.Setup(p.A, p.pitchA, m0, p.m, p.k);
+    ob.Setup(p.B, p.pitchB, n0, p.n, p.k);
+    // A: scales [m][2 ceil(k/64)] when stored K-contiguous, else pairs-major; B the same way
+    const bool forA = t < BT;
+    const int srow = forA ? min(m0 + t, p.m - 1) : min(n0 + t - BT, p.n - 1);
+    const auto loadScales = [&](int stage) {
+        return forA ? LoadScales(p.scaleA, !AK, p.m, srow, stage, p.k)
+                    : LoadScales(p.scaleB, !BK, p.n, srow, stage, p.k);
+    };
+
+    f32x4 acc[kF][kF];
+#pragma unroll
+    for (int i = 0; i < kF; ++i) {
+#pragma unroll
+        for (int j = 0; j < kF; ++j) {
+            acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    }
+    u32x4 va[OpA::kLoads], vb[OpB::kLoads];
+    uint32_t vs = 0;
+    const auto load = [&](int stage) {
+        oa.Load(stage, va);
+        ob.Load(stage, vb);
+        if (t < 2 * BT) {
+            vs = loadScales(stage);
+        }
+    };
+    const auto store = [&](int buf) {
+        oa.Store(sA[buf], va);
+        ob.Store(sB[buf], vb);
+        if (t < 2 * BT) {
+            sS[buf][t] = vs;
+        }
+    };
+    const int stages = (p.k + kStepK - 1) / kStepK;
+    if (stages > 0) {
+        load(0);
+        store(0);
+    }
+    __syncthreads();
+    for (int s = 0; s < stages; ++s) {
+        const int buf = s & 1;
+        if (s + 1 < stages) {
+            load(s + 1);
+        }
+        ZeroBlocks<OpA, FP4, AK, BT / 2>(sA[buf], wm, lane, [&](int r) { return sS[buf][r]; });
+        ZeroBlocks<OpB, FP4, BK, BT / 2>(sB[buf], wn, lane, [&](int r) { return sS[buf][BT + r]; });
+        i32x8 b[kF];
+        uint32_t sb[kF];
+#pragma unroll
+        for (int j = 0; j < kF; ++j) {
+            b[j] = OpB::Fragment(sB[buf], wn + 16 * j, lane);
+            sb[j] = sS[buf][BT + wn + 16 * j + r16] >> (8 * g);
+        }
+#pragma unroll
+        for (int i = 0; i < kF; ++i) {
+            const i32x8 a = OpA::Fragment(sA[buf], wm + 16 * i, lane);
+            const uint32_t sa = sS[buf][wm + 16 * i + r16] >> (8 * g);
+            // transposed product: a lane holds four consecutive columns of D
+#pragma unroll
+            for (int j = 0; j < kF; ++j) {
+                acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                    b[j], a, acc[i][j], kFmt, kFmt, 0, static_cast<int>(sb[j]), 0, static_cast<int>(sa));
+            }
+        }
+        if (s + 1 < stages) {
+            store(buf ^ 1);
+        }
+        __syncthreads();
+    }
+    StoreTiles<kF, kF>(p, acc, m0 + wm, n0 + wn, lane);
+}
+
+// The same tile with direct-to-LDS loads: a ring of four stages, three in
+// flight (two stages where the largest FP8 tile fills LDS with them).  Both operands' and the
+// scales' chunks go straight to LDS; a last partial stage is loaded through
+// registers with zero fill.  Needs 16-byte aligned operand rows (and whole
+// chunks per row where they are row-contiguous) and 2-byte aligned scales.
+template <bool FP4, bool AK, bool BK, int BT>
+__global__ __launch_bounds__(Threads(BT)) void LtMxDmaKernel(MxArgs p)
+{
+    constexpr int kFmt = FP4 ? 4 : 0;
+    constexpr int kFA = BT / 32;               // 16-row fragments per wave
+    constexpr int kFB = BT / WavesN(BT) / 16;
+    constexpr int kWaves = Threads(BT) / 64;
+    // four stages while they fit, of the largest FP8 tile two
+    constexpr int kStages = BT == 256 && !FP4 ? 2 : 4;
+    using OpA = Operand<FP4, AK, BT>;
+    using OpB = Operand<FP4, BK, BT>;
+    // scales: [A, B][block pair of the stage][row], one pair per dword
+    constexpr int kScaleLoads = 4 * BT / 64 / kWaves;
+    constexpr int kPerStage = OpA::kLoads + OpB::kLoads + kScaleLoads;
+    struct Stage {
+        uint8_t a[OpA::kBytes];
+        uint8_t b[OpB::kBytes];
+        uint32_t s[2][2][BT];
+    };
+    __shared__ __attribute__((aligned(1024))) Stage ring[kStages];
+
+    int m0, n0;
+    TileOf<BT>(p, m0, n0);
+    const int t = static_cast<int>(threadIdx.x);
+    const int lane = t & 63;
+    const int wave = dev::Uniform(t >> 6);
+    const int wm = (wave / WavesN(BT)) * (BT / 2);
+    const int wn = (wave % WavesN(BT)) * (BT / WavesN(BT));
+    const int r16 = lane & 15;
+    const int g = lane >> 4;
+    const int nFull = p.k / kStepK;
+    const int stages = (p.k + kStepK - 1) / kStepK;
+
+    OpA oa;
+    OpB ob;
+    oa.SetupDma(p.A, p.pitchA, m0, p.m);
+    ob.SetupDma(p.B, p.pitchB, n0, p.n);
+    const int pairs = (p.k + 63) / 64;
+    const uint8_t* ssrc[kScaleLoads];
+    long long sstep[kScaleLoads];
+#pragma unroll
+    for (int y = 0; y < kScaleLoads; ++y) {
+        const int idx = 64 * (wave + kWaves * y) + lane;
+        const bool forA = idx < 2 * BT;
+        const int h = (idx / BT) & 1;
+        const bool pairsMajor = forA ? !AK : !BK;
+        const int rows = forA ? p.m : p.n;
+        const int row = min((forA ? m0 : n0) + idx % BT, rows - 1);
+        ssrc[y] = (forA ? p.scaleA : p.scaleB) +
+                  2 * (pairsMajor ? static_cast<long long>(min(h, pairs - 1)) * rows + row
+                                  : static_cast<long long>(row) * pairs + min(h, pairs - 1));
+        sstep[y] = pairsMajor ? 4ll * rows : 4;
+    }
+    const auto issue = [&](int s) {
+        Stage& st = ring[s % kStages];
+        if (s < nFull) {
+            oa.Issue(s, st.a, wave);
+            ob.Issue(s, st.b, wave);
+            const uint32_t base = dev::LdsAddr(&st.s[0][0][0]);
+#pragma unroll
+            for (int y = 0; y < kScaleLoads; ++y) {
+                LdsDma2(ssrc[y] + s * sstep[y],
+                        __builtin_amdgcn_readfirstlane(base + 256u * (wave + kWaves * y)));
+            }
+        } else {
+            OpA ta;
+            OpB tb;
+            ta.Setup(p.A, p.pitchA, m0, p.m, p.k);
+            tb.Setup(p.B, p.pitchB, n0, p.n, p.k);
+            u32x4 va[OpA::kLoads], vb[OpB::kLoads];
+            ta.Load(s, va);
+            tb.Load(s, vb);
+            ta.Store(st.a, va);
+            tb.Store(st.b, vb);
+            if (t < 2 * BT) {  // 256 or 512 threads: one row each
+                const bool forA = t < BT;
+                const int row = forA ? min(m0 + t, p.m - 1) : min(n0 + t - BT, p.n - 1);
+                const uint32_t v = forA ? LoadScales(p.scaleA, !AK, p.m, row, s, p.k)
+                                        : LoadScales(p.scaleB, !BK, p.n, row, s, p.k);
+                st.s[forA ? 0 : 1][0][t % BT] = v & 0xFFFFu;
+                st.s[forA ? 0 : 1][1][t % BT] = v >> 16;
+            }
+        }
+    };
+
+    f32x4 acc[kFA][kFB];
+#pragma unroll
+    for (int i = 0; i < kFA; ++i) {
+#pragma unroll
+        for (int j = 0; j < kFB; ++j) {
+            acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    }
+    for (int s = 0; s < kStages - 1 && s < stages; ++s) {
+        issue(s);
+    }
+    for (int s = 0; s < stages; ++s) {
+        // this wave's stages after s may stay in flight
+        const int pending = kStages == 2 ? 0 : (s + 1 < nFull ? 1 : 0) + (s + 2 < nFull ? 1 : 0);
+        if (pending == 2) {
+            dev::WaitVmcnt<2 * kPerStage>();
+        } else if (pending == 1) {
+            dev::WaitVmcnt<kPerStage>();
+        } else {
+            dev::WaitVmcnt<0>();
+        }
+        dev::BarrierLds();
+        Stage& st = ring[s % kStages];
+        // the next loads go out before the products, which do not wait for them
+        if (s + kStages - 1 < stages) {
+            issue(s + kStages - 1);
+        }
+        ZeroBlocks<OpA, FP4, AK, BT / 2>(st.a, wm, lane,
+                                         [&](int r) { return st.s[0][0][r] | (st.s[0][1][r] << 16); });
+        ZeroBlocks<OpB, FP4, BK, BT / WavesN(BT)>(st.b, wn, lane,
+                                                  [&](int r) { return st.s[1][0][r] | (st.s[1][1][r] << 16); });
+        i32x8 b[kFB];
+        uint32_t sb[kFB];
+#pragma unroll
+        for (int j = 0; j < kFB; ++j) {
+            b[j] = OpB::Fragment(st.b, wn + 16 * j, lane);
+            sb[j] = st.s[1][g >> 1][wn + 16 * j + r16] >> (8 * (g & 1));
+        }
+#pragma unroll
+        for (int i = 0; i < kFA; ++i) {
+            const i32x8 a = OpA::Fragment(st.a, wm + 16 * i, lane);
+            const uint32_t sa = st.s[0][g >> 1][wm + 16 * i + r16] >> (8 * (g & 1));
+#pragma unroll
+            for (int j = 0; j < kFB; ++j) {
+                acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                    b[j], a, acc[i][j], kFmt, kFmt, 0, static_cast<int>(sb[j]), 0, static_cast<int>(sa));
+            }
+        }
+    }
+    StoreTiles<kFA, kFB>(p, acc, m0 + wm, n0 + wn, lane);
+}
+
+template <bool FP4, bool AK, bool BK>
+void Launch(hipStream_t st, MxArgs p)
+{
+    // Largest tiles that still give (about) every CU one: larger tiles need
+    // fewer LDS bytes per product, fewer tiles leave CUs idle.  MXFP8 NT: 4096^3
+    // 84 us with 256 tiles (156 with 128); 2048^3 54 us with 256 and 29 with
+    // 128 tiles; 1024 x 1024 x 4096 37 us with 128 and 20 with 64.
+    const auto tiles = [&](int bt) {
+        p.tilesM = (p.m + bt - 1) / bt;
+        p.tilesN = (p.n + bt - 1) / bt;
+        return static_cast<long long>(p.tilesM) * p.tilesN;
+    };
+    if (p.dma != 0 && tiles(256) >= 192) {
+        const dim3 grid(static_cast<unsigned>(tiles(256)));
+        hipLaunchKernelGGL((LtMxDmaKernel<FP4, AK, BK, 256>), grid, dim3(Threads(256)), 0, st, p);
+        return;
+    }
+    const bool big = tiles(128) >= 256;
+    const dim3 grid(static_cast<unsigned>(tiles(big ? 128 : 64)));
+    if (p.dma != 0) {
+        if (big) {
+            hipLaunchKernelGGL((LtMxDmaKernel<FP4, AK, BK, 128>), grid, dim3(256), 0, st, p);
+        } else {
+            hipLaunchKernelGGL((LtMxDmaKernel<FP4, AK, BK, 64>), grid, dim3(256), 0, st, p);
+        }
+    } else {
+        if (big) {
+            hipLaunchKernelGGL((LtMxKernel<FP4, AK, BK, 128>), grid, dim3(256), 0, st, p);
+        } else {
+            hipLaunchKernelGGL((LtMxKernel<FP4, AK, BK, 64>), grid, dim3(256), 0, st, p);
+        }
+    }
+}
+
+template <bool FP4>
+void LaunchTrans(hipStream_t st, bool aK, bool bK, const MxArgs& p)
+{
+    if (aK) {
+        bK ? Launch<FP4, true, true>(st, p) : Launch<FP4, true, false>(st, p);
+    } else {
+        bK ? Launch<FP4, false, true>(st, p) : Launch<FP4, false, false>(st, p);
     }
 }
 
@@ -280,25 +740,24 @@ aclblasStatus_t LtMxLaunch(hipStream_t st, bool fp4, bool transA, bool transB, i
     p.k = k;
     p.ldc = ldc;
     p.ldd = ldd;
-    p.transA = transA ? 1 : 0;
-    p.transB = transB ? 1 : 0;
-    p.vecA = (reinterpret_cast<uintptr_t>(A) % 16 == 0 && p.pitchA % 16 == 0) ? 1 : 0;
-    p.vecB = (reinterpret_cast<uintptr_t>(B) % 16 == 0 && p.pitchB % 16 == 0) ? 1 : 0;
+    p.vecC = (C != nullptr && reinterpret_cast<uintptr_t>(C) % 16 == 0 && ldc % 4 == 0) ? 1 : 0;
+    p.vecD = (reinterpret_cast<uintptr_t>(D) % (bf16Out ? 8 : 16) == 0 && ldd % 4 == 0) ? 1 : 0;
+    p.bf16Out = bf16Out ? 1 : 0;
+    // direct-to-LDS: aligned rows, and row-contiguous rows of whole 16-byte chunks
+    const int rowAlign = fp4 ? 32 : 16;
+    const bool alignedOps = reinterpret_cast<uintptr_t>(A) % 16 == 0 && lda % 16 == 0 &&
+                            reinterpret_cast<uintptr_t>(B) % 16 == 0 && ldb % 16 == 0;
+    p.dma = (alignedOps && (!transA || m % rowAlign == 0) && (transB || n % rowAlign == 0) &&
+             reinterpret_cast<uintptr_t>(scaleA) % 2 == 0 && reinterpret_cast<uintptr_t>(scaleB) % 2 == 0)
+                ? 1
+                : 0;
     p.alpha = alpha;
     p.beta = beta;
-    const dim3 grid((n + kTile - 1) / kTile, (m + kTile - 1) / kTile);
+    // A is K-contiguous when it is not transposed, B when it is
     if (fp4) {
-        if (bf16Out) {
-            hipLaunchKernelGGL((LtMxKernel<true, true>), grid, dim3(kThreads), 0, st, p);
-        } else {
-            hipLaunchKernelGGL((LtMxKernel<true, false>), grid, dim3(kThreads), 0, st, p);
-        }
+        LaunchTrans<true>(st, !transA, transB, p);
     } else {
-        if (bf16Out) {
-            hipLaunchKernelGGL((LtMxKernel<false, true>), grid, dim3(kThreads), 0, st, p);
-        } else {
-            hipLaunchKernelGGL((LtMxKernel<false, false>), grid, dim3(kThreads), 0, st, p);
-        }
+        LaunchTrans<false>(st, !transA, transB, p);
     }
     return LaunchStatus("aclblasLtMatmul");
 }

@@ -202,3 +202,41 @@ def test_fp32_distinct_c_and_d(lt, trans):
                        ldc, ldd)
     _check(res, gold, M, N, O.LT_FP32)
     np.testing.assert_allclose(res[:, :N], gold[:, :N], rtol=1e-5, atol=1e-4)
+
+
+def _mx_slice(stored, scales, fp4, rows, k, k_rows, lo, hi):
+    """Rows lo..hi of an operand and its scales.  k_rows: stored K by row (rows along the fast axis)."""
+    pairs = (k + 63) // 64
+    if k_rows:
+        data = stored[:, lo // 2:(hi + 1) // 2] if fp4 else stored[:, lo:hi]
+        sc = scales.reshape(pairs, rows, 2)[:, lo:hi]
+    else:
+        data, sc = stored[lo:hi], scales.reshape(rows, 2 * pairs)[lo:hi]
+    return np.ascontiguousarray(data), np.ascontiguousarray(sc).reshape(-1)
+
+
+@pytest.mark.parametrize("fp4", [False, True], ids=["mxfp8", "mxfp4"])
+@pytest.mark.parametrize("trans", ["NN", "NT", "TN", "TT"])
+@pytest.mark.parametrize("m,n", [(3616, 3616), (2048, 2080), (130, 96)])
+def test_mx_tiles_agree(lt, fp4, trans, m, n):
+    """Every tile size (256, 128, 64; ragged edges, a last K block alone in its stage, zero scale bytes) gives the
+    bits of the smallest one, on corner blocks of the product: the sum over K runs in the same stages."""
+    rng = np.random.default_rng(m + n + fp4)
+    k, (ta, tb) = 416, trans
+    typ = O.LT_MXFP4 if fp4 else O.LT_MXFP8
+    A, lda = _mx_operand(rng, *((m, k) if ta == "N" else (k, m)), fp4)
+    W, ldb = _mx_operand(rng, *((k, n) if tb == "N" else (n, k)), fp4)
+    sA = rng.integers(120, 135, size=_scale_bytes(m, k, ta != "N")).astype(np.uint8)
+    sW = rng.integers(120, 135, size=_scale_bytes(n, k, tb == "N")).astype(np.uint8)
+    sA[rng.integers(0, sA.size, 50)] = 0
+    sW[rng.integers(0, sW.size, 50)] = 0
+    st, full = _run(lt, typ, B.ACL_FLOAT, ta, tb, m, n, k, 1.0, 0.0, A, lda, W, ldb, sA, sW, None, n, n)
+    assert st == 0
+    for r0, r1 in ((0, 62), (m - 66, m)):
+        for c0, c1 in ((0, 60), (n - 62, n)):
+            a, sa = _mx_slice(A, sA, fp4, m, k, ta == "T", r0, r1)
+            w, sw = _mx_slice(W, sW, fp4, n, k, tb == "N", c0, c1)
+            st, part = _run(lt, typ, B.ACL_FLOAT, ta, tb, r1 - r0, c1 - c0, k, 1.0, 0.0, a, a.shape[1], w, w.shape[1],
+                            sa, sw, None, c1 - c0, c1 - c0)
+            assert st == 0
+            assert np.array_equal(full[r0:r1, c0:c1], part)

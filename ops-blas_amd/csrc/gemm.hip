@@ -152,14 +152,8 @@ aclblasStatus_t RunGemm(const _aclblas_handle* h, int ka, int kb, int ok, bool t
     // alignment of batched pointers is re-checked per problem on the device
     const void* a0 = Aarr != nullptr ? nullptr : A;
     const void* b0 = Barr != nullptr ? nullptr : B;
-    const void* c0 = Carr != nullptr ? nullptr : C;
     p.vecA = Aligned16(a0, lda, ElemBytes(ka)) ? 1 : 0;
     p.vecB = Aligned16(b0, ldb, ElemBytes(kb)) ? 1 : 0;
-    {
-        const int cb = ok == kOutF32 ? 4 : 2;  // bytes per C element; four move together
-        p.vecC = (reinterpret_cast<uintptr_t>(c0) % (4 * cb) == 0 && (static_cast<long long>(ldc) * cb) % (4 * cb) == 0)
-                     ? 1 : 0;
-    }
     const hipStream_t st = h->stream;
     const int cus = h->cu_count > 0 ? h->cu_count : 256;
     const int eb = ElemBytes(ka);

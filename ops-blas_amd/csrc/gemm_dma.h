@@ -109,22 +109,46 @@ struct DmaSource {
     }
 };
 
-// Register-path load of stage s of one operand (bounds-checked, zero fill):
-// used for the stages of a final partial 64-k pair.
+// Eight consecutive 16-bit values at p, `valid` of them readable (the rest
+// zero); any alignment.
+__device__ __forceinline__ uint4 LoadChunk16(const uint16_t* p, int valid)
+{
+    if (valid >= 8) {
+        const auto v = *(const ACL_GLOBAL U32x4Any*)p;
+        return make_uint4(v.x, v.y, v.z, v.w);
+    }
+    uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        if (e < valid) {
+            w[e / 2] |= static_cast<uint32_t>(dev::LoadG<uint16_t>(p + e)) << (16 * (e & 1));
+        }
+    }
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// Register-path load of stage s of one operand (bounds-checked, zero fill), a
+// 16-byte chunk at a time: used for the stages of a final partial 64-k pair,
+// and for every stage of an operand the DMA cannot read.
 template <bool MM>
 __device__ __forceinline__ void FillStage(uint8_t* buf, const uint16_t* X, int ld, int row0, int rows, int s, int K,
                                           int t)
 {
-    for (int e = t; e < 256 * kKS; e += kThreads) {
-        const int r = MM ? (e & 255) : (e >> 5);
-        const int kk = MM ? (e >> 8) : (e & 31);
-        const int k = StageK(s, kk);
-        uint16_t v = 0;
-        if (row0 + r < rows && k < K) {
-            v = MM ? X[static_cast<size_t>(k) * ld + row0 + r] : X[static_cast<size_t>(row0 + r) * ld + k];
-        }
-        const uint32_t off = MM ? MmOffset(kk, r >> 3) + 2u * (r & 7) : KmOffset(r, kk >> 3) + 2u * (kk & 7);
-        *reinterpret_cast<uint16_t*>(buf + off) = v;
+    constexpr int kChunks = 256 * kKS / 8 / kThreads;
+    uint4 v[kChunks];
+#pragma unroll
+    for (int q = 0; q < kChunks; ++q) {
+        const int e = t + q * kThreads;
+        // M-major: row kk, chunk e % 32 of 8 indices; K-major: row e / 4, chunk e % 4 of 8 k
+        const int k = MM ? StageK(s, e >> 5) : StageK(s, 8 * (e & 3));
+        const int r = row0 + (MM ? 8 * (e & 31) : e >> 2);
+        const int valid = MM ? (k < K ? rows - r : 0) : (r < rows ? K - k : 0);
+        v[q] = LoadChunk16(X + (MM ? static_cast<size_t>(k) * ld + r : static_cast<size_t>(r) * ld + k), valid);
+    }
+#pragma unroll
+    for (int q = 0; q < kChunks; ++q) {
+        const int e = t + q * kThreads;
+        *reinterpret_cast<uint4*>(buf + (MM ? MmOffset(e >> 5, e & 31) : KmOffset(e >> 2, e & 3))) = v[q];
     }
 }
 
@@ -143,39 +167,30 @@ __device__ __forceinline__ uint32_t TrBase(int wbase, int lane)
 
 }  // namespace dma
 
-// 256 x 256 tile of one problem (no batch), both operands 16-bit (KA),
-// direct-to-LDS loads.  AMM: op(A) stored m-contiguous (A not transposed);
-// BMM: op(B) stored n-contiguous (B transposed).  The host launches it only
-// when A, B and their leading dimensions are 16-byte aligned.
+// 256 x 256 tile of one problem, both operands 16-bit (KA).  AMM: op(A) stored
+// m-contiguous (A not transposed); BMM: op(B) stored n-contiguous (B
+// transposed).  direct: the operands can be read by the DMA (16-byte aligned
+// bases and leading dimensions, whole chunks along an index-contiguous
+// operand); otherwise every stage is loaded through registers.
 template <int KA, int OK, bool AMM, bool BMM>
-__global__ __launch_bounds__(dma::kThreads) void GemmDmaKernel(GemmArgs p)
+__device__ __forceinline__ void GemmDmaTile(const TileJob& q, bool direct, int m0, int n0, uint8_t (*lds)[2][dma::kOpBytes])
 {
     using namespace dma;
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[kStages][2][kOpBytes];
-
-    int bid = blockIdx.x;
-    if (gridDim.x % 8 == 0) {
-        bid = (bid % 8) * (gridDim.x / 8) + bid / 8;
-    }
-    int tm, tn;
-    TileOf(bid, p.tilesM, p.tilesN, p.group, tm, tn);
-    const int m0 = tm * kBM;
-    const int n0 = tn * kBN;
     const int t = threadIdx.x;
     const int lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = (wave % kWGM) * (kBM / kWGM);
     const int wn = (wave / kWGM) * (kBN / kWGN);
-    const uint16_t* A = static_cast<const uint16_t*>(p.A);
-    const uint16_t* B = static_cast<const uint16_t*>(p.B);
-    const int K = p.k;
-    const int nFull = 2 * (K / 64);
+    const uint16_t* A = reinterpret_cast<const uint16_t*>(q.A);
+    const uint16_t* B = reinterpret_cast<const uint16_t*>(q.B);
+    const int K = q.k;
+    const int nFull = direct ? 2 * (K / 64) : 0;
     const int nst = 2 * ((K + 63) / 64);
 
     DmaSource da;
     DmaSource db;
-    da.Setup<AMM>(A, p.lda, m0, p.m, wave, lane);
-    db.Setup<BMM>(B, p.ldb, n0, p.n, wave, lane);
+    da.Setup<AMM>(A, q.lda, m0, q.m, wave, lane);
+    db.Setup<BMM>(B, q.ldb, n0, q.n, wave, lane);
 
     auto issue = [&](int s) {
         uint8_t* bufA = lds[s % kStages][0];
@@ -184,8 +199,8 @@ __global__ __launch_bounds__(dma::kThreads) void GemmDmaKernel(GemmArgs p)
             da.Issue(s, bufA, wave);
             db.Issue(s, bufB, wave);
         } else {
-            FillStage<AMM>(bufA, A, p.lda, m0, p.m, s, K, t);
-            FillStage<BMM>(bufB, B, p.ldb, n0, p.n, s, K, t);
+            FillStage<AMM>(bufA, A, q.lda, m0, q.m, s, K, t);
+            FillStage<BMM>(bufB, B, q.ldb, n0, q.n, s, K, t);
         }
     };
 
@@ -255,15 +270,6 @@ __global__ __launch_bounds__(dma::kThreads) void GemmDmaKernel(GemmArgs p)
         dev::SetPriority<0>();
     }
 
-    TileJob q;
-    q.C = p.C;
-    q.m = p.m;
-    q.n = p.n;
-    q.k = p.k;
-    q.ldc = p.ldc;
-    q.vecC = p.vecC != 0;
-    q.alpha = p.alpha;
-    q.beta = p.beta;
     StoreTileC<OK, TM, TN, false>(q, acc, m0 + wm, n0 + wn, lane);
 }
 
@@ -479,7 +485,6 @@ __global__ __launch_bounds__(dma::kThreads) void GemmDmaFp8Kernel(GemmArgs p)
     q.n = p.n;
     q.k = p.k;
     q.ldc = p.ldc;
-    q.vecC = p.vecC != 0;
     float alpha = p.alpha;
     if (p.scaleA != nullptr) alpha *= *p.scaleA;
     if (p.scaleB != nullptr) alpha *= *p.scaleB;
@@ -553,16 +558,21 @@ template <bool MM>
 __device__ __forceinline__ void FillStage2(uint8_t* buf, const uint16_t* X, int ld, int row0, int rows, int s, int K,
                                            int t)
 {
-    for (int e = t; e < 256 * kKS; e += dma::kThreads) {
-        const int r = MM ? (e & 255) : (e >> 6);
-        const int kk = MM ? (e >> 8) : (e & 63);
-        const int k = kKS * s + kk;
-        uint16_t v = 0;
-        if (row0 + r < rows && k < K) {
-            v = MM ? X[static_cast<size_t>(k) * ld + row0 + r] : X[static_cast<size_t>(row0 + r) * ld + k];
-        }
-        const uint32_t off = MM ? Mm2Offset(kk, r >> 3) + 2u * (r & 7) : SwizzledOffset(r, 2 * kk);
-        *reinterpret_cast<uint16_t*>(buf + off) = v;
+    constexpr int kChunks = 256 * kKS / 8 / dma::kThreads;
+    uint4 v[kChunks];
+#pragma unroll
+    for (int q = 0; q < kChunks; ++q) {
+        const int e = t + q * dma::kThreads;
+        const int k = kKS * s + (MM ? e >> 5 : 8 * (e & 7));
+        const int r = row0 + (MM ? 8 * (e & 31) : e >> 3);
+        const int valid = MM ? (k < K ? rows - r : 0) : (r < rows ? K - k : 0);
+        v[q] = dma::LoadChunk16(X + (MM ? static_cast<size_t>(k) * ld + r : static_cast<size_t>(r) * ld + k), valid);
+    }
+#pragma unroll
+    for (int q = 0; q < kChunks; ++q) {
+        const int e = t + q * dma::kThreads;
+        *reinterpret_cast<uint4*>(buf + (MM ? Mm2Offset(e >> 5, e & 31) : SwizzledOffset(e >> 3, 16 * (e & 7)))) =
+            v[q];
     }
 }
 
@@ -579,34 +589,24 @@ __device__ __forceinline__ uint32_t Tr2Base(int wbase, int lane)
 }  // namespace dma2
 
 template <int KA, int OK, bool AMM, bool BMM>
-__global__ __launch_bounds__(dma::kThreads) void GemmDma64Kernel(GemmArgs p)
+__device__ __forceinline__ void GemmDma64Tile(const TileJob& q, bool direct, int m0, int n0, uint8_t (*lds)[2][dma2::kOpBytes])
 {
     using namespace dma2;
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[kStages][2][kOpBytes];
-
-    int bid = blockIdx.x;
-    if (gridDim.x % 8 == 0) {
-        bid = (bid % 8) * (gridDim.x / 8) + bid / 8;
-    }
-    int tm, tn;
-    TileOf(bid, p.tilesM, p.tilesN, p.group, tm, tn);
-    const int m0 = tm * dma::kBM;
-    const int n0 = tn * dma::kBN;
     const int t = threadIdx.x;
     const int lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = (wave % dma::kWGM) * (dma::kBM / dma::kWGM);
     const int wn = (wave / dma::kWGM) * (dma::kBN / dma::kWGN);
-    const uint16_t* A = static_cast<const uint16_t*>(p.A);
-    const uint16_t* B = static_cast<const uint16_t*>(p.B);
-    const int K = p.k;
-    const int nFull = K / kKS;
+    const uint16_t* A = reinterpret_cast<const uint16_t*>(q.A);
+    const uint16_t* B = reinterpret_cast<const uint16_t*>(q.B);
+    const int K = q.k;
+    const int nFull = direct ? K / kKS : 0;
     const int nst = (K + kKS - 1) / kKS;
 
     DmaSource2 da;
     DmaSource2 db;
-    da.Setup<AMM>(A, p.lda, m0, p.m, wave, lane);
-    db.Setup<BMM>(B, p.ldb, n0, p.n, wave, lane);
+    da.Setup<AMM>(A, q.lda, m0, q.m, wave, lane);
+    db.Setup<BMM>(B, q.ldb, n0, q.n, wave, lane);
 
     auto issue = [&](int s) {
         uint8_t* bufA = lds[s % kStages][0];
@@ -615,8 +615,8 @@ __global__ __launch_bounds__(dma::kThreads) void GemmDma64Kernel(GemmArgs p)
             da.Issue(s, bufA, wave);
             db.Issue(s, bufB, wave);
         } else {
-            FillStage2<AMM>(bufA, A, p.lda, m0, p.m, s, K, t);
-            FillStage2<BMM>(bufB, B, p.ldb, n0, p.n, s, K, t);
+            FillStage2<AMM>(bufA, A, q.lda, m0, q.m, s, K, t);
+            FillStage2<BMM>(bufB, B, q.ldb, n0, q.n, s, K, t);
         }
     };
 
@@ -682,16 +682,99 @@ __global__ __launch_bounds__(dma::kThreads) void GemmDma64Kernel(GemmArgs p)
         dev::SetPriority<0>();
     }
 
+    StoreTileC<OK, TM, TN, false>(q, acc, m0 + wm, n0 + wn, lane);
+}
+
+// Whether the DMA can read both operands of a job.
+template <bool AMM, bool BMM>
+__device__ __forceinline__ bool Direct(const TileJob& q)
+{
+    return q.vecA && q.vecB && (!AMM || q.m % 8 == 0) && (!BMM || q.n % 8 == 0);
+}
+
+// Which of the two 16-bit pipelines a tile runs: m-contiguous A 32-k stages
+// (transposing reads, conflict-free), k-contiguous A 64-k stages (128-byte
+// rows, conflict-free).
+template <int KA, int OK, bool AMM, bool BMM>
+__device__ __forceinline__ void GemmDmaAny(const TileJob& q, int m0, int n0, uint8_t* lds)
+{
+    const bool direct = Direct<AMM, BMM>(q);
+    if constexpr (AMM) {
+        GemmDmaTile<KA, OK, AMM, BMM>(q, direct, m0, n0, reinterpret_cast<uint8_t (*)[2][dma::kOpBytes]>(lds));
+    } else {
+        GemmDma64Tile<KA, OK, AMM, BMM>(q, direct, m0, n0, reinterpret_cast<uint8_t (*)[2][dma2::kOpBytes]>(lds));
+    }
+}
+constexpr int kDmaLdsBytes = dma::kStages * 2 * dma::kOpBytes;
+static_assert(kDmaLdsBytes == dma2::kStages * 2 * dma2::kOpBytes, "both pipelines use the same LDS");
+
+// One problem, or a uniform batch through pointer arrays: one workgroup per
+// 256 x 256 tile.
+template <int KA, int OK, bool AMM, bool BMM>
+__global__ __launch_bounds__(dma::kThreads) void GemmDmaKernel(GemmArgs p)
+{
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[kDmaLdsBytes];
+    int bid = blockIdx.x;
+    if (gridDim.x % 8 == 0) {
+        bid = (bid % 8) * (gridDim.x / 8) + bid / 8;
+    }
+    const int tilesPer = p.tilesM * p.tilesN;
+    const int prob = bid / tilesPer;
+    int tm, tn;
+    TileOf(bid - prob * tilesPer, p.tilesM, p.tilesN, p.group, tm, tn);
     TileJob q;
-    q.C = p.C;
+    q.A = static_cast<const uint8_t*>(p.Aarr != nullptr ? p.Aarr[prob] : p.A);
+    q.B = static_cast<const uint8_t*>(p.Barr != nullptr ? p.Barr[prob] : p.B);
+    q.C = p.Carr != nullptr ? p.Carr[prob] : p.C;
     q.m = p.m;
     q.n = p.n;
     q.k = p.k;
+    q.lda = p.lda;
+    q.ldb = p.ldb;
     q.ldc = p.ldc;
-    q.vecC = p.vecC != 0;
+    // per-problem pointers of a batch may be less aligned than the host assumed
+    q.vecA = p.vecA && (reinterpret_cast<uintptr_t>(q.A) % 16 == 0);
+    q.vecB = p.vecB && (reinterpret_cast<uintptr_t>(q.B) % 16 == 0);
     q.alpha = p.alpha;
     q.beta = p.beta;
-    StoreTileC<OK, TM, TN, false>(q, acc, m0 + wm, n0 + wn, lane);
+    GemmDmaAny<KA, OK, AMM, BMM>(q, tm * dma::kBM, tn * dma::kBN, lds);
+}
+
+// Grouped 16-bit GEMM: one workgroup per 256 x 256 tile of the problems of one
+// transpose pair (ordered by decreasing k on the host, so the longest tiles
+// start first and the hardware's dispatch balances the rest; a persistent grid
+// would fix each CU's tiles in advance).  Thirty-two consecutive tiles run on
+// one XCD at a time, so that its L2 shares their operands.  A, B and C come from
+// the device pointer arrays by the record's slot.
+template <int KA, int OK, bool AMM, bool BMM>
+__global__ __launch_bounds__(dma::kThreads) void GroupedDmaKernel(const GroupedProblem* __restrict__ probs,
+                                                                 int numProbs, const void* const* __restrict__ Aarr,
+                                                                 const void* const* __restrict__ Barr,
+                                                                 void* const* __restrict__ Carr)
+{
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[kDmaLdsBytes];
+    int tile = static_cast<int>(blockIdx.x);
+    if ((tile | 255) < static_cast<int>(gridDim.x)) {
+        tile = (tile & ~255) + (tile & 7) * 32 + ((tile & 255) >> 3);
+    }
+    const GroupedProblem& g = probs[ProblemOf(probs, numProbs, tile)];
+    int tm, tn;
+    TileOf(tile - g.tileStart, g.tilesM, g.tilesN, kGroupedL2Rows, tm, tn);
+    TileJob q;
+    q.A = static_cast<const uint8_t*>(Aarr[g.slot]);
+    q.B = static_cast<const uint8_t*>(Barr[g.slot]);
+    q.C = Carr[g.slot];
+    q.m = g.m;
+    q.n = g.n;
+    q.k = g.k;
+    q.lda = g.lda;
+    q.ldb = g.ldb;
+    q.ldc = g.ldc;
+    q.vecA = g.vecA != 0 && reinterpret_cast<uintptr_t>(q.A) % 16 == 0;
+    q.vecB = g.vecB != 0 && reinterpret_cast<uintptr_t>(q.B) % 16 == 0;
+    q.alpha = g.alpha;
+    q.beta = g.beta;
+    GemmDmaAny<KA, OK, AMM, BMM>(q, tm * dma::kBM, tn * dma::kBN, lds);
 }
 
 }  // namespace gemm

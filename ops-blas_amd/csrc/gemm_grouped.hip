@@ -138,7 +138,6 @@ extern "C" aclblasStatus_t aclblasSgemmGroupedBatched(
             p.beta = beta;
             p.vecA = Aligned16(p.A, p.lda) ? 1 : 0;
             p.vecB = Aligned16(p.B, p.ldb) ? 1 : 0;
-            p.vecC = Aligned16(p.C, p.ldc) ? 1 : 0;
             if (p.k > 0 && (p.A == nullptr || p.B == nullptr)) {
                 LogError("aclblasSgemmGroupedBatched", "null A/B matrix in group %d", g);
                 return ACLBLAS_STATUS_INVALID_VALUE;
@@ -281,6 +280,32 @@ void LaunchGroupedEx(hipStream_t st, int tile, unsigned grid, const GroupedProbl
     }
 }
 
+// pair: 2 transA + transB.
+template <int KA, int OK>
+void LaunchGroupedDirect(hipStream_t st, int pair, unsigned grid, const GroupedProblem* table, int count,
+                         const void* const* A, const void* const* B, void* const* C)
+{
+    const dim3 block(gemm::dma::kThreads);
+    switch (pair) {
+        case 0:
+            hipLaunchKernelGGL((gemm::GroupedDmaKernel<KA, OK, true, false>), dim3(grid), block, 0, st, table, count,
+                               A, B, C);
+            break;
+        case 1:
+            hipLaunchKernelGGL((gemm::GroupedDmaKernel<KA, OK, true, true>), dim3(grid), block, 0, st, table, count,
+                               A, B, C);
+            break;
+        case 2:
+            hipLaunchKernelGGL((gemm::GroupedDmaKernel<KA, OK, false, false>), dim3(grid), block, 0, st, table, count,
+                               A, B, C);
+            break;
+        default:
+            hipLaunchKernelGGL((gemm::GroupedDmaKernel<KA, OK, false, true>), dim3(grid), block, 0, st, table, count,
+                               A, B, C);
+            break;
+    }
+}
+
 }  // namespace
 }  // namespace aclblas
 
@@ -365,7 +390,6 @@ extern "C" aclblasStatus_t aclblasGemmGroupedBatchedEx(
                     // leading-dimension part of the alignment test (pointers on the device)
                     p.vecA = (static_cast<long long>(p.lda) * ea) % 16 == 0 ? 1 : 0;
                     p.vecB = (static_cast<long long>(p.ldb) * eb) % 16 == 0 ? 1 : 0;
-                    p.vecC = (static_cast<long long>(p.ldc) * 2) % 16 == 0 ? 1 : 0;
                     probs.push_back(p);
                 }
             }
@@ -388,14 +412,54 @@ extern "C" aclblasStatus_t aclblasGemmGroupedBatchedEx(
     const tune::Choice c = tune::Get(handle, tune::kOpGrouped, tune::GroupedBucket(1, tiles128, cus),
                                      tune::Choice{kDefaultTile, kDefaultBlocksPerCu});
     const int tile = c.a;
-    long long tiles = 0;
-    for (GroupedProblem& p : probs) {
-        p.tilesM = (p.m + tile - 1) / tile;
-        p.tilesN = (p.n + tile - 1) / tile;
-        p.tileStart = static_cast<int>(tiles);
-        tiles += static_cast<long long>(p.tilesM) * p.tilesN;
-        if (tiles > 0x7FFFFFFFll) {
-            LogError("aclblasGemmGroupedBatchedEx", "more than 2^31 tiles");
+    // 16-bit problems whose leading dimensions the DMA can read go to the
+    // direct-to-LDS kernel, one launch per transpose pair, when their 256 tiles
+    // occupy half the CUs or more and pad the work by at most a quarter over 128
+    // tiles; the rest to the persistent kernel.  64 shapes up to 2048 (padding
+    // 1.12) 557 -> 384 us; 64 shapes up to 512 (1.39) would take 45 instead of 39.
+    // A launch choice forced on the handle keeps the persistent kernel.
+    const bool sixteen = Atype == ACL_FLOAT16 || Atype == ACL_BF16;
+    const auto part = [&](const GroupedProblem& p) {
+        const bool direct = sixteen && p.vecA != 0 && p.vecB != 0 && (p.transA != 0 || p.m % 8 == 0) &&
+                            (p.transB == 0 || p.n % 8 == 0);
+        return direct ? 2 * p.transA + p.transB : 4;
+    };
+    const auto tilesOf = [](const GroupedProblem& p, int edge) {
+        return static_cast<long long>((p.m + edge - 1) / edge) * ((p.n + edge - 1) / edge);
+    };
+    long long direct256 = 0;
+    double work256 = 0.0;
+    double work128 = 0.0;
+    for (const GroupedProblem& p : probs) {
+        if (part(p) < 4) {
+            direct256 += tilesOf(p, 256);
+            work256 += 4.0 * p.k * tilesOf(p, 256);
+            work128 += 1.0 * p.k * tilesOf(p, 128);
+        }
+    }
+    const bool useDirect = handle->tune_override[tune::kOpGrouped][0] == 0 && 2 * direct256 >= cus &&
+                           work256 <= 1.25 * work128;
+    if (useDirect) {
+        std::stable_sort(probs.begin(), probs.end(),
+                         [&](const GroupedProblem& x, const GroupedProblem& y) { return part(x) < part(y); });
+    }
+    struct Segment {
+        int first = 0;
+        int count = 0;
+        long long tiles = 0;
+    } seg[5];
+    for (size_t i = 0; i < probs.size(); ++i) {
+        GroupedProblem& p = probs[i];
+        Segment& sg = seg[useDirect ? part(p) : 4];
+        const int edge = useDirect && part(p) < 4 ? 256 : tile;
+        sg.first = sg.count == 0 ? static_cast<int>(i) : sg.first;
+        sg.count++;
+        p.tilesM = (p.m + edge - 1) / edge;
+        p.tilesN = (p.n + edge - 1) / edge;
+        p.tileStart = static_cast<int>(sg.tiles);
+        sg.tiles += tilesOf(p, edge);
+        if (sg.tiles > (edge == 256 ? 0x7FFFFFll : 0x7FFFFFFFll)) {
+            LogError("aclblasGemmGroupedBatchedEx", "too many tiles");
             return ACLBLAS_STATUS_NOT_SUPPORTED;
         }
     }
@@ -404,13 +468,28 @@ extern "C" aclblasStatus_t aclblasGemmGroupedBatchedEx(
     if (st != ACLBLAS_STATUS_SUCCESS) {
         return st;
     }
-    const long long cap = static_cast<long long>(cus) * c.b;
-    const unsigned grid = static_cast<unsigned>(tiles < cap ? tiles : cap);
     const auto* table = static_cast<const GroupedProblem*>(dev);
-    const int count = static_cast<int>(probs.size());
-    const int nt = static_cast<int>(tiles);
     const hipStream_t s = handle->stream;
     using namespace gemm;
+    for (int d = 0; d < 4; ++d) {
+        if (seg[d].count > 0) {
+            if (Atype == ACL_FLOAT16) {
+                LaunchGroupedDirect<kF16, kOutF16A>(s, d, static_cast<unsigned>(seg[d].tiles), table + seg[d].first,
+                                                    seg[d].count, Aarray, Barray, Carray);
+            } else {
+                LaunchGroupedDirect<kBF16, kOutBF16>(s, d, static_cast<unsigned>(seg[d].tiles), table + seg[d].first,
+                                                     seg[d].count, Aarray, Barray, Carray);
+            }
+        }
+    }
+    if (seg[4].count == 0) {
+        return LaunchStatus("aclblasGemmGroupedBatchedEx");
+    }
+    table += seg[4].first;
+    const int count = seg[4].count;
+    const int nt = static_cast<int>(seg[4].tiles);
+    const long long cap = static_cast<long long>(cus) * c.b;
+    const unsigned grid = static_cast<unsigned>(nt < cap ? nt : cap);
     const bool a4 = Atype == ACL_FLOAT8_E4M3FN;
     const bool b4 = Btype == ACL_FLOAT8_E4M3FN;
     if (Atype == ACL_FLOAT16) {

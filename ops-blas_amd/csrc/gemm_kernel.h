@@ -77,6 +77,11 @@ constexpr int kRowBytes = 128;   // one k-block per LDS row
 constexpr int kThreads = 256;     // default workgroup: 2 x 2 waves
 constexpr int kWaveSize = 64;
 
+// Vectors of 16 and 8 bytes at any address (the hardware's global accesses
+// need no alignment).
+typedef uint32_t U32x4Any __attribute__((ext_vector_type(4), aligned(1)));
+typedef uint32_t U32x2Any __attribute__((ext_vector_type(2), aligned(1)));
+
 struct GemmArgs {
     const void* A;
     const void* B;
@@ -87,8 +92,7 @@ struct GemmArgs {
     float alpha, beta;
     const float* scaleA;    // optional device scalars multiplying op(A), op(B)
     const float* scaleB;
-    int vecA, vecB;         // 1 when 16-byte vector loads are legal
-    int vecC;               // 1 when four consecutive C elements can move as one vector
+    int vecA, vecB;         // 1 when base and leading dimension are 16-byte aligned (the DMA kernels need it)
     int tilesM, tilesN;
     int group;              // tile rows per L2 group (TileOf)
     // batched form: device arrays of per-problem pointers (A/B/C unused), or null
@@ -148,14 +152,25 @@ struct TileLoader {
         }
     }
 
-    // All chunks of k-block kb in range and 16-byte aligned.
+    // Sixteen bytes at any alignment the element type allows (the hardware's
+    // global loads take any address): operands whose base or leading dimension
+    // is not a multiple of 16 bytes used to be read element by element, 4 times
+    // slower over a ragged 16-bit group (64 odd shapes up to 2048: 2320 us, 775 us
+    // now).
+    __device__ __forceinline__ static uint4 LoadAny(const uint8_t* p)
+    {
+        const auto v = *(const ACL_GLOBAL U32x4Any*)p;
+        return make_uint4(v.x, v.y, v.z, v.w);
+    }
+
+    // All chunks of k-block kb in range.
     __device__ __forceinline__ void FetchFull(int kb) { FetchFullInto(kb, v); }
     __device__ __forceinline__ void FetchFullInto(int kb, uint4 (&dst)[kPerThread]) const
     {
         const uint8_t* p = base + static_cast<size_t>(kb) * kstep;
 #pragma unroll
         for (int q = 0; q < kPerThread; ++q) {
-            dst[q] = dev::LoadG<uint4>(p + q * qstride);
+            dst[q] = LoadAny(p + q * qstride);
         }
     }
 
@@ -231,7 +246,7 @@ struct TileLoader {
     __device__ __forceinline__ static uint4 LoadChunk(const uint8_t* p, bool full, int valid)
     {
         if (full) {
-            return dev::LoadG<uint4>(p);
+            return LoadAny(p);
         }
         uint32_t w[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
@@ -243,13 +258,12 @@ struct TileLoader {
         return make_uint4(w[0], w[1], w[2], w[3]);
     }
 
-    __device__ __forceinline__ void Fetch(const uint8_t* X, int ld, bool kcontig, bool vec, int r0, int rlim,
-                                          int k0, int klim)
+    __device__ __forceinline__ void Fetch(const uint8_t* X, int ld, bool kcontig, int r0, int rlim, int k0, int klim)
     {
-        FetchInto(X, ld, kcontig, vec, r0, rlim, k0, klim, v);
+        FetchInto(X, ld, kcontig, r0, rlim, k0, klim, v);
     }
-    __device__ __forceinline__ void FetchInto(const uint8_t* X, int ld, bool kcontig, bool vec, int r0, int rlim,
-                                              int k0, int klim, uint4 (&v)[kPerThread]) const
+    __device__ __forceinline__ void FetchInto(const uint8_t* X, int ld, bool kcontig, int r0, int rlim, int k0,
+                                              int klim, uint4 (&v)[kPerThread]) const
     {
         const int t = threadIdx.x;
         if (kcontig) {
@@ -261,7 +275,7 @@ struct TileLoader {
                 const int gk = k0 + (id % (kRowBytes / 16)) * E;
                 const uint8_t* p = X + (static_cast<size_t>(gr) * ld + gk) * EB;
                 const int valid = gr < rlim ? klim - gk : 0;
-                v[q] = LoadChunk(p, vec && valid >= E, valid);
+                v[q] = LoadChunk(p, valid >= E, valid);
             }
         } else {
             const int mc = t % kMChunks;
@@ -272,7 +286,7 @@ struct TileLoader {
                 const int gk = k0 + kg * kPerThread + q;
                 const uint8_t* p = X + (static_cast<size_t>(gk) * ld + gr) * EB;
                 const int valid = gk < klim ? rlim - gr : 0;
-                v[q] = LoadChunk(p, vec && valid >= E, valid);
+                v[q] = LoadChunk(p, valid >= E, valid);
             }
         }
     }
@@ -545,10 +559,13 @@ __device__ __forceinline__ void LoadC4(const void* C, size_t idx, bool full, int
 {
     if (full) {
         if (OK == kOutF32) {
-            const float4 x = dev::LoadG<float4>(static_cast<const float*>(C) + idx);
-            c[0] = x.x; c[1] = x.y; c[2] = x.z; c[3] = x.w;
+            const auto x = *(const ACL_GLOBAL U32x4Any*)(static_cast<const float*>(C) + idx);
+            c[0] = __uint_as_float(x.x);
+            c[1] = __uint_as_float(x.y);
+            c[2] = __uint_as_float(x.z);
+            c[3] = __uint_as_float(x.w);
         } else {
-            const uint2 x = dev::LoadG<uint2>(static_cast<const uint16_t*>(C) + idx);
+            const auto x = *(const ACL_GLOBAL U32x2Any*)(static_cast<const uint16_t*>(C) + idx);
             const uint16_t h[4] = {static_cast<uint16_t>(x.x), static_cast<uint16_t>(x.x >> 16),
                                    static_cast<uint16_t>(x.y), static_cast<uint16_t>(x.y >> 16)};
 #pragma unroll
@@ -565,16 +582,16 @@ __device__ __forceinline__ void StoreC4(void* C, size_t idx, bool full, int vali
 {
     if (full) {
         if (OK == kOutF32) {
-            dev::StoreG(static_cast<float*>(C) + idx, make_float4(v[0], v[1], v[2], v[3]));
+            *(ACL_GLOBAL U32x4Any*)(static_cast<float*>(C) + idx) =
+                U32x4Any{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
         } else {
             uint16_t h[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 h[e] = OK == kOutBF16 ? ToBf16(v[e]) : (OK == kOutF16A ? ToF16Away(v[e]) : ToF16(v[e]));
             }
-            dev::StoreG(static_cast<uint16_t*>(C) + idx,
-                        make_uint2(h[0] | (static_cast<uint32_t>(h[1]) << 16),
-                                   h[2] | (static_cast<uint32_t>(h[3]) << 16)));
+            *(ACL_GLOBAL U32x2Any*)(static_cast<uint16_t*>(C) + idx) =
+                U32x2Any{h[0] | (static_cast<uint32_t>(h[1]) << 16), h[2] | (static_cast<uint32_t>(h[3]) << 16)};
         }
         return;
     }
@@ -608,7 +625,7 @@ struct TileJob {
     int m, n, k;
     int lda, ldb, ldc;
     bool aK, bK;            // operand tiles are k-contiguous in memory
-    bool vecA, vecB, vecC;  // 16-byte operand loads / 4-element C moves are legal
+    bool vecA, vecB;        // operands the DMA can read (16-byte aligned)
     float alpha, beta;
 };
 
@@ -637,7 +654,7 @@ __device__ __forceinline__ void StoreTileC(const TileJob& q, const f32x4 (&acc)[
             for (int e = 0; e < 4; ++e) {
                 v[e] = alpha * acc[i][j][e];
             }
-            const bool full = q.vecC && row + 4 <= q.m;
+            const bool full = row + 4 <= q.m;
             if (beta != 0.0f) {
                 float c[4];
                 LoadC4<OK>(q.C, base, full, q.m - row, c);
@@ -675,7 +692,7 @@ __device__ __forceinline__ void PreloadTileC(const TileJob& q, int row0, int col
             const bool in = col < q.n && row < q.m;
             // rows past m or columns past n read element (0, 0) and are never stored
             const size_t base = in ? static_cast<size_t>(col) * q.ldc + row : 0;
-            LoadC4<OK>(q.C, base, in && q.vecC && row + 4 <= q.m, in ? q.m - row : 1, c[i][j]);
+            LoadC4<OK>(q.C, base, in && row + 4 <= q.m, in ? q.m - row : 1, c[i][j]);
         }
     }
 }
@@ -704,7 +721,7 @@ __device__ __forceinline__ void StoreTileCPre(const TileJob& q, const f32x4 (&ac
             for (int e = 0; e < 4; ++e) {
                 v[e] = alpha * acc[i][j][e] + beta * c[i][j][e];
             }
-            StoreC4<OK>(q.C, base, q.vecC && row + 4 <= q.m, q.m - row, v);
+            StoreC4<OK>(q.C, base, row + 4 <= q.m, q.m - row, v);
         }
     }
 }
@@ -787,8 +804,8 @@ __device__ __forceinline__ void GemmTile(const TileJob& q, int m0, int n0, uint8
     lb.Setup(q.B, q.ldb, q.bK, n0);
     // interior tiles take the unchecked path for every full k-block
     const int fullK = q.k / kK;
-    const bool interiorA = q.vecA && m0 + BM <= q.m;
-    const bool interiorB = q.vecB && n0 + BN <= q.n;
+    const bool interiorA = m0 + BM <= q.m;
+    const bool interiorB = n0 + BN <= q.n;
 
     f32x4 acc[TM][TN];
 #pragma unroll
@@ -801,12 +818,12 @@ __device__ __forceinline__ void GemmTile(const TileJob& q, int m0, int n0, uint8
         if (interiorA && kb < fullK) {
             la.FetchFull(kb);
         } else {
-            la.Fetch(q.A, q.lda, q.aK, q.vecA, m0, q.m, kb * kK, q.k);
+            la.Fetch(q.A, q.lda, q.aK, m0, q.m, kb * kK, q.k);
         }
         if (interiorB && kb < fullK) {
             lb.FetchFull(kb);
         } else {
-            lb.Fetch(q.B, q.ldb, q.bK, q.vecB, n0, q.n, kb * kK, q.k);
+            lb.Fetch(q.B, q.ldb, q.bK, n0, q.n, kb * kK, q.k);
         }
     };
     if (nk > 0) {
@@ -878,8 +895,8 @@ __device__ __forceinline__ void GemmTileDeep(const TileJob& q, int m0, int n0, u
     la.Setup(q.A, q.lda, q.aK, m0);
     lb.Setup(q.B, q.ldb, q.bK, n0);
     const int fullK = q.k / kK;
-    const bool interiorA = q.vecA && m0 + BM <= q.m;
-    const bool interiorB = q.vecB && n0 + BN <= q.n;
+    const bool interiorA = m0 + BM <= q.m;
+    const bool interiorB = n0 + BN <= q.n;
 
     f32x4 acc[TM][TN];
 #pragma unroll
@@ -901,12 +918,12 @@ __device__ __forceinline__ void GemmTileDeep(const TileJob& q, int m0, int n0, u
         if (interiorA && kb < fullK) {
             la.FetchFullInto(kb, da);
         } else {
-            la.FetchInto(q.A, q.lda, q.aK, q.vecA, m0, q.m, kb * kK, q.k, da);
+            la.FetchInto(q.A, q.lda, q.aK, m0, q.m, kb * kK, q.k, da);
         }
         if (interiorB && kb < fullK) {
             lb.FetchFullInto(kb, db);
         } else {
-            lb.FetchInto(q.B, q.ldb, q.bK, q.vecB, n0, q.n, kb * kK, q.k, db);
+            lb.FetchInto(q.B, q.ldb, q.bK, n0, q.n, kb * kK, q.k, db);
         }
     };
     const int fr = lane & 15;
@@ -1022,7 +1039,6 @@ __global__ __launch_bounds__(kWaveSize * WGM * WGN) void GemmKernel(GemmArgs p)
     // per-problem pointers of a batch may be less aligned than the host assumed
     q.vecA = p.vecA && (reinterpret_cast<uintptr_t>(q.A) % 16 == 0);
     q.vecB = p.vecB && (reinterpret_cast<uintptr_t>(q.B) % 16 == 0);
-    q.vecC = p.vecC && (reinterpret_cast<uintptr_t>(q.C) % 16 == 0);
     float alpha = p.alpha;
     if (p.scaleA != nullptr) alpha *= *p.scaleA;
     if (p.scaleB != nullptr) alpha *= *p.scaleB;
@@ -1046,9 +1062,27 @@ struct GroupedProblem {
     float alpha, beta;
     int tilesM, tilesN;
     int tileStart;          // first global tile index of this problem
-    int vecA, vecB, vecC;
+    int vecA, vecB;
     int slot;               // index into the device pointer arrays (when the launch passes them)
 };
+
+// The problem that holds a tile: the last whose tileStart is at most it.  A
+// wave compares 64 records at a time (one round trip; a binary search's six
+// dependent ones took 6 us before a tile's first load).
+__device__ __forceinline__ int ProblemOf(const GroupedProblem* probs, int numProbs, int tile)
+{
+    int last = 0;
+    for (int base = 0; base < numProbs; base += kWaveSize) {
+        const int i = base + (static_cast<int>(threadIdx.x) & 63);
+        const bool before = i < numProbs && dev::G(&probs[min(i, numProbs - 1)].tileStart)[0] <= tile;
+        const int count = __builtin_popcountll(__builtin_amdgcn_ballot_w64(before));
+        last = base + count - 1;
+        if (count < kWaveSize) {
+            break;
+        }
+    }
+    return __builtin_amdgcn_readfirstlane(last);
+}
 
 // L2 group height of the grouped kernel's tile walk (problems are small: a
 // few tile rows each).
@@ -1056,8 +1090,7 @@ constexpr int kGroupedL2Rows = 8;
 
 // Persistent grouped GEMM: the grid strides over the concatenated tile lists
 // of all problems (problems ordered by decreasing k on the host, so the
-// longest tiles start first); each workgroup finds its problem by binary
-// search over tileStart.
+// longest tiles start first).
 // With device pointer arrays (Aarr != nullptr) a record's A, B and C come from
 // Aarr/Barr/Carr[slot], and its vector flags hold only the leading-dimension
 // part of the alignment test: the pointers are checked here.
@@ -1071,17 +1104,7 @@ __global__ __launch_bounds__(kThreads) void GroupedGemmKernel(const GroupedProbl
     __shared__ __attribute__((aligned(16))) uint8_t sA[2][BM * kRowBytes];
     __shared__ __attribute__((aligned(16))) uint8_t sB[2][BN * kRowBytes];
     for (int tile = blockIdx.x; tile < totalTiles; tile += gridDim.x) {
-        int lo = 0;
-        int hi = numProbs - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (probs[mid].tileStart <= tile) {
-                lo = mid;
-            } else {
-                hi = mid - 1;
-            }
-        }
-        const GroupedProblem& g = probs[lo];
+        const GroupedProblem& g = probs[ProblemOf(probs, numProbs, tile)];
         int tm, tn;
         TileOf(tile - g.tileStart, g.tilesM, g.tilesN, kGroupedL2Rows, tm, tn);
         TileJob q;
@@ -1098,14 +1121,12 @@ __global__ __launch_bounds__(kThreads) void GroupedGemmKernel(const GroupedProbl
         q.bK = g.transB == 0;
         q.vecA = g.vecA != 0;
         q.vecB = g.vecB != 0;
-        q.vecC = g.vecC != 0;
         if (Aarr != nullptr) {
             q.A = static_cast<const uint8_t*>(Aarr[g.slot]);
             q.B = static_cast<const uint8_t*>(Barr[g.slot]);
             q.C = Carr[g.slot];
             q.vecA = q.vecA && (reinterpret_cast<uintptr_t>(q.A) % 16 == 0);
             q.vecB = q.vecB && (reinterpret_cast<uintptr_t>(q.B) % 16 == 0);
-            q.vecC = q.vecC && (reinterpret_cast<uintptr_t>(q.C) % 16 == 0);
         }
         q.alpha = g.alpha;
         q.beta = g.beta;
@@ -1139,25 +1160,23 @@ inline void LaunchGemmTyped(hipStream_t st, GemmArgs p, int batch, int tile, int
     constexpr int EB = KindInfo<KA>::bytes;
     p.group = group;
     if constexpr (KA == kBF16 || KA == kF16) {
-        // direct-to-LDS kernel: one problem, 16-byte aligned operands, and an
-        // index-contiguous operand's extent a whole number of 16-byte chunks
-        // (its DMA copies whole chunks: a partial last chunk would read past
-        // the end of the operand's last column)
-        if (tile == 256 && p.Aarr == nullptr && p.vecA != 0 && p.vecB != 0 && DmaExtentsWhole(p, 8)) {
+        // direct-to-LDS kernel: 16-byte aligned operands (a batch's pointers are
+        // checked on the device), and an index-contiguous operand's extent a
+        // whole number of 16-byte chunks (its DMA copies whole chunks: a partial
+        // last chunk would read past the end of the operand's last column)
+        if (tile == 256 && p.vecA != 0 && p.vecB != 0 && DmaExtentsWhole(p, 8)) {
             p.tilesM = (p.m + 255) / 256;
             p.tilesN = (p.n + 255) / 256;
-            const dim3 grid(p.tilesM * p.tilesN);
+            const dim3 grid(p.tilesM * p.tilesN * batch);
             const dim3 block(dma::kThreads);
-            // m-contiguous A: 32-k stages (transposing reads, conflict-free);
-            // k-contiguous A: 64-k stages (128-byte rows, conflict-free)
             if (p.transA == 0 && p.transB == 0) {
                 hipLaunchKernelGGL((GemmDmaKernel<KA, OK, true, false>), grid, block, 0, st, p);
             } else if (p.transA == 0) {
                 hipLaunchKernelGGL((GemmDmaKernel<KA, OK, true, true>), grid, block, 0, st, p);
             } else if (p.transB == 0) {
-                hipLaunchKernelGGL((GemmDma64Kernel<KA, OK, false, false>), grid, block, 0, st, p);
+                hipLaunchKernelGGL((GemmDmaKernel<KA, OK, false, false>), grid, block, 0, st, p);
             } else {
-                hipLaunchKernelGGL((GemmDma64Kernel<KA, OK, false, true>), grid, block, 0, st, p);
+                hipLaunchKernelGGL((GemmDmaKernel<KA, OK, false, true>), grid, block, 0, st, p);
             }
             return;
         }

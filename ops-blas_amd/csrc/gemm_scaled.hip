@@ -284,11 +284,6 @@ extern "C" aclblasStatus_t aclblasGemmExScaled(
     p.scaleB = scaleB;
     p.vecA = (reinterpret_cast<uintptr_t>(A) % 16 == 0 && lda % 16 == 0) ? 1 : 0;
     p.vecB = (reinterpret_cast<uintptr_t>(B) % 16 == 0 && ldb % 16 == 0) ? 1 : 0;
-    {
-        const int cb = ok == kOutF32 ? 4 : 2;
-        p.vecC = (reinterpret_cast<uintptr_t>(C) % (4 * cb) == 0 && (static_cast<long long>(ldc) * cb) % (4 * cb) == 0)
-                     ? 1 : 0;
-    }
     const int cus = handle->cu_count > 0 ? handle->cu_count : 256;
     const long long t128 = static_cast<long long>((m + 127) / 128) * ((n + 127) / 128);
     const tune::Choice c = tune::Get(handle, tune::kOpGemm, tune::GemmBucket(tune::kClassF8Scaled, t128, k, cus),

@@ -141,7 +141,7 @@ void LaunchGetrf(const _aclblas_handle* h, float* const* A, int n, int lda, int*
         LaunchGetrfWave<PIVOT>(st, A, n, lda, ipiv, info, batch, WaveRows(h, n, batch));
     } else if (n <= 256) {
         const int cus = h->cu_count > 0 ? h->cu_count : 256;
-        LaunchGetrfBlocked<PIVOT>(st, A, n, lda, ipiv, info, batch, batch < 2 * cus ? batch : 2 * cus);
+        LaunchGetrfBlocked<PIVOT>(st, A, n, lda, ipiv, info, batch, cus);
     } else if (n <= kMaxLargeN) {
         LaunchGetrfLarge<PIVOT>(st, A, n, lda, ipiv, info, batch);
     } else {

@@ -35,36 +35,52 @@ using lub::kWaves;
 
 // Rows k0.. of columns 0..k0-1 take the panel's interchanges: position q
 // receives the row the panel's map names for it.  Wave v permutes columns
-// v, v + 4, ...; a lane reads all its rows of a column before writing any.
+// v, v + 4, ..., kCols of them at a time so that their loads are in flight
+// together; a lane reads all its rows of a column before writing any.
+template <int N>
 __device__ __forceinline__ void PermuteLeft(float* A, int ld, int n, int k0, const int* map)
 {
+    constexpr int kRows = N / dev::kWave;
+    constexpr int kCols = 4;
     const int lane = dev::LaneId();
     const int wave = static_cast<int>(threadIdx.x) / dev::kWave;
     const int rows = n - k0;
-    for (int c = wave; c < k0; c += kWaves) {
-        float* col = A + static_cast<size_t>(c) * ld + k0;
-        float v[4];
-        dev::StaticFor<0, 4>([&](auto ic) {
-            constexpr int i = decltype(ic)::value;
-            const int q = lane + 64 * i;
-            v[i] = q < rows ? col[map[q]] : 0.0f;
+    int from[kRows];
+    dev::StaticFor<0, kRows>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        from[i] = map[min(lane + 64 * i, rows - 1)];
+    });
+    const auto col = dev::G(A) + k0;
+    for (int c = wave; c < k0; c += kCols * kWaves) {
+        float v[kCols][kRows];
+        dev::StaticFor<0, kCols>([&](auto cc) {
+            constexpr int q = decltype(cc)::value;
+            const size_t at = static_cast<size_t>(min(c + q * kWaves, k0 - 1)) * ld;
+            dev::StaticFor<0, kRows>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                v[q][i] = col[at + from[i]];
+            });
         });
-        dev::StaticFor<0, 4>([&](auto ic) {
-            constexpr int i = decltype(ic)::value;
-            const int q = lane + 64 * i;
-            if (q < rows) {
-                col[q] = v[i];
-            }
+        dev::StaticFor<0, kCols>([&](auto cc) {
+            constexpr int q = decltype(cc)::value;
+            const size_t at = static_cast<size_t>(c + q * kWaves) * ld;
+            dev::StaticFor<0, kRows>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                if (c + q * kWaves < k0 && lane + 64 * i < rows) {
+                    col[at + lane + 64 * i] = v[q][i];
+                }
+            });
         });
     }
 }
 
-template <bool PIVOT>
-__global__ __launch_bounds__(kThreads, 2) void GetrfBlockedKernel(float* const* __restrict__ Aarray, int n, int lda,
-                                                                 int* __restrict__ ipiv, int* __restrict__ info,
-                                                                 int batch)
+// N: the largest order of the instance; PER: workgroups per CU it is built for.
+template <bool PIVOT, int N, int PER>
+__global__ __launch_bounds__(kThreads, PER) void GetrfBlockedKernel(float* const* __restrict__ Aarray, int n, int lda,
+                                                                   int* __restrict__ ipiv, int* __restrict__ info,
+                                                                   int batch)
 {
-    __shared__ __attribute__((aligned(16))) lub::FactorShared<0> sh;
+    __shared__ __attribute__((aligned(16))) lub::FactorShared<0, N> sh;
     const int t = threadIdx.x;
     for (int b = blockIdx.x; b < batch; b += gridDim.x) {
         float* const Ab = Aarray[b];
@@ -72,18 +88,18 @@ __global__ __launch_bounds__(kThreads, 2) void GetrfBlockedKernel(float* const* 
         int infoVal = 0;
         for (int k0 = 0; k0 < n; k0 += kNb) {
             int wl = 0;
-            const int z = lub::FactorPanel<0, PIVOT, true>(view, k0, nullptr, sh, &wl);
+            const int z = lub::FactorPanel<0, PIVOT, true, N>(view, k0, nullptr, sh, &wl);
             if (PIVOT) {
                 const int count = z != 0 ? wl + 1 : wl;
                 if (t < count) {
                     ipiv[static_cast<size_t>(b) * n + k0 + t] = k0 + sh.pw[t] + 1;
                 }
             }
-            lub::PanelInverses<0>(view, k0, wl, nullptr, sh);
+            lub::PanelInverses<0, N>(view, k0, wl, nullptr, sh);
             __syncthreads();
-            lub::SweepTrailing<0>(view, k0, sh);
+            lub::SweepTrailing<0, N>(view, k0, sh);
             if (PIVOT) {
-                PermuteLeft(view.LU, lda, n, k0, sh.rowmap);
+                PermuteLeft<N>(view.LU, lda, n, k0, sh.rowmap);
             }
             __syncthreads();
             if (z != 0) {
@@ -99,10 +115,29 @@ __global__ __launch_bounds__(kThreads, 2) void GetrfBlockedKernel(float* const* 
 
 }  // namespace
 
-template <bool PIVOT>
-void LaunchGetrfBlocked(hipStream_t st, float* const* A, int n, int lda, int* ipiv, int* info, int batch, int grid)
+template <bool PIVOT, int N, int PER>
+void Launch(hipStream_t st, float* const* A, int n, int lda, int* ipiv, int* info, int batch, int cus)
 {
-    hipLaunchKernelGGL((GetrfBlockedKernel<PIVOT>), dim3(grid), dim3(kThreads), 0, st, A, n, lda, ipiv, info, batch);
+    const int grid = batch < PER * cus ? batch : PER * cus;
+    hipLaunchKernelGGL((GetrfBlockedKernel<PIVOT, N, PER>), dim3(grid), dim3(kThreads), 0, st, A, n, lda, ipiv, info,
+                       batch);
+}
+
+template <bool PIVOT>
+void LaunchGetrfBlocked(hipStream_t st, float* const* A, int n, int lda, int* ipiv, int* info, int batch, int cus)
+{
+    // Both the column chain of a panel and the memory round trips of a sweep
+    // leave a CU idle, so the instance for the order at hand (less LDS, fewer
+    // accumulators) puts more workgroups on it.  2048 x 128: 590 us with the
+    // 256 instance (two per CU, left columns permuted one at a time), 445 us
+    // with three per CU, 370 us with four.
+    if (n <= 128) {
+        Launch<PIVOT, 128, 4>(st, A, n, lda, ipiv, info, batch, cus);
+    } else if (n <= 192) {
+        Launch<PIVOT, 192, 3>(st, A, n, lda, ipiv, info, batch, cus);
+    } else {
+        Launch<PIVOT, 256, 2>(st, A, n, lda, ipiv, info, batch, cus);
+    }
 }
 
 template void LaunchGetrfBlocked<true>(hipStream_t, float* const*, int, int, int*, int*, int, int);

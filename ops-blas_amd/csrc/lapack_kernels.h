@@ -16,9 +16,9 @@ void LaunchGetrfWave(hipStream_t st, float* const* A, int n, int lda, int* ipiv,
 void LaunchGetrfWaveOutOfPlace(hipStream_t st, const float* const* A, int n, int lda, float* out, float** table,
                                int* ipiv, int* info, int batch, int rows);
 
-// LU, 64 < n <= 256, blocked (getrf_blocked.hip); grid: persistent workgroups
+// LU, 64 < n <= 256, blocked (getrf_blocked.hip); cus: compute units
 template <bool PIVOT>
-void LaunchGetrfBlocked(hipStream_t st, float* const* A, int n, int lda, int* ipiv, int* info, int batch, int grid);
+void LaunchGetrfBlocked(hipStream_t st, float* const* A, int n, int lda, int* ipiv, int* info, int batch, int cus);
 
 // LU, 256 < n <= kMaxLargeN, blocked over many workgroups per matrix (getrf_large.hip)
 constexpr int kMaxLargeN = 2048;

@@ -28,7 +28,6 @@ constexpr int kNb = 32;                  // panel width
 constexpr int kThreads = 256;            // four waves
 constexpr int kWaves = kThreads / kWave;
 constexpr int kTileN = 16;               // sweep tile width
-constexpr int kMaxTiles = kMaxN / 16;    // 16-row accumulator tiles per column tile
 constexpr int kLd = kNb + 4;             // row stride (floats) of 32-wide FP32 LDS blocks: 16-byte rows
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -74,23 +73,27 @@ __device__ __forceinline__ void SplitPlanes(float x, uint16_t (&h)[P])
     });
 }
 
+// N: the largest order an instance takes (a multiple of 32, at most kMaxN).  It
+// sizes the LDS and the accumulators of a sweep tile, and so the workgroups
+// that share a CU.
+
 // -L21 and U12 of the current panel in the operand format of the update.
-template <int P>
+template <int P, int N>
 struct UpdateOperands {  // P BF16 planes each
-    alignas(16) uint16_t l[P][kMaxN - kNb][kNb];          // -L21 [plane][row][k]
+    alignas(16) uint16_t l[P][N - kNb][kNb];              // -L21 [plane][row][k]
     alignas(16) uint16_t u[kWaves][P][kTileN][kNb];       // U12^T per wave [plane][col][k]
 };
-template <>
-struct UpdateOperands<0> {  // FP32
-    alignas(16) float l[kMaxN - kNb][kLd];                // -L21 [row][k]
+template <int N>
+struct UpdateOperands<0, N> {  // FP32
+    alignas(16) float l[N - kNb][kLd];                    // -L21 [row][k]
     alignas(16) float u[kWaves][kTileN][kLd];             // U12^T per wave [col][k]
 };
 
-template <int P>
+template <int P, int N = kMaxN>
 struct FactorShared {
     alignas(16) float cand[2][kWaves][kNb];               // each wave's best row, by column parity
     alignas(16) uint64_t cand64[2][kWaves];               // its packed key (PackCand), 0: no candidate
-    int rowmap[kMaxN];                                    // panel row map (position -> row, relative)
+    int rowmap[N];                                        // panel row map (position -> row, relative)
     int pw[kNb];                                          // pivot position chosen at each panel column
     int zero;                                             // zero-pivot column of a one-wave panel
     alignas(16) float linv[kNb][kLd];                     // inv(L11), row-major
@@ -100,7 +103,7 @@ struct FactorShared {
         alignas(16) float l11[kNb][kLd];                  // panel rows 0..31: L11 below, U11 on/above the diagonal
         alignas(16) float ut[kWaves][kNb][kTileN + 1];    // per-wave top rows of the sweep tile
     };
-    UpdateOperands<P> op;
+    UpdateOperands<P, N> op;
 };
 
 // A wave's best candidate as one integer whose maximum over the waves is the
@@ -137,8 +140,8 @@ __device__ __forceinline__ void WaveSync()
 // from j on are zero, so a sweep with this panel applies exactly those j steps
 // to the trailing columns.  Returns the zero-pivot column + 1, or 0 (*wl =
 // width then).  Uniform over the workgroup; ends with a barrier.
-template <int P, bool PIVOT, bool DIVIDE>
-__device__ __forceinline__ int FactorPanel(const PanelView& pv, int k0, int* gmap, FactorShared<P>& sh, int* wl)
+template <int P, bool PIVOT, bool DIVIDE, int N>
+__device__ __forceinline__ int FactorPanel(const PanelView& pv, int k0, int* gmap, FactorShared<P, N>& sh, int* wl)
 {
     const int n = pv.n;
     const size_t ld = static_cast<size_t>(pv.ld);
@@ -251,11 +254,13 @@ __device__ __forceinline__ int FactorPanel(const PanelView& pv, int k0, int* gma
             if constexpr (DIVIDE) {
                 // the reference's multipliers; rows left alone keep their exact values
                 const float l = a[j] / pivot;
-                a[j] = upd ? l : a[j];
-                dev::StaticFor<j + 1, kNb>([&](auto cc) {
-                    constexpr int c = decltype(cc)::value;
-                    a[c] = upd ? fmaf(-l, u[c], a[c]) : a[c];
-                });
+                if (upd) {
+                    a[j] = l;
+                    dev::StaticFor<j + 1, kNb>([&](auto cc) {
+                        constexpr int c = decltype(cc)::value;
+                        a[c] = fmaf(-l, u[c], a[c]);
+                    });
+                }
             } else {
                 // rows left alone get l = 0: a - 0 * u keeps their value (up to the sign of a zero, and
                 // for finite u), which is all the backward-error-checked solve needs
@@ -337,8 +342,8 @@ __device__ __forceinline__ int FactorPanel(const PanelView& pv, int k0, int* gma
 // block is the identity's: the panel wrote zeros there; rows and columns past
 // the panel's width are the identity's too).  It
 // goes to LDS (for U12) and, when g is given, to g (32 x 32, column-major).
-template <int P>
-__device__ __forceinline__ void PanelInverses(const PanelView& pv, int k0, int wl, float* g, FactorShared<P>& sh)
+template <int P, int N>
+__device__ __forceinline__ void PanelInverses(const PanelView& pv, int k0, int wl, float* g, FactorShared<P, N>& sh)
 {
     const int lane = dev::LaneId();
     const int wave = static_cast<int>(threadIdx.x) / kWave;
@@ -378,12 +383,13 @@ __device__ __forceinline__ void PanelInverses(const PanelView& pv, int k0, int w
 // One 16-column tile of the trailing matrix in accumulators: element j of
 // accumulator t of a lane holds row 16t + (lane & 15) (panel position) and
 // column c0 + 4 (lane >> 4) + j.
-typedef f32x4 SweepAcc[kMaxTiles];
+template <int N>
+using SweepAcc = f32x4[N / 16];
 
 // Gathers the tile at column c0 through the panel's row map.
-template <int P>
-__device__ __forceinline__ void GatherTile(const PanelView& pv, int k0, int c0, const FactorShared<P>& sh,
-                                           SweepAcc& acc)
+template <int P, int N>
+__device__ __forceinline__ void GatherTile(const PanelView& pv, int k0, int c0, const FactorShared<P, N>& sh,
+                                           SweepAcc<N>& acc)
 {
     const int n = pv.n;
     const size_t ld = static_cast<size_t>(pv.srcLd);
@@ -393,7 +399,7 @@ __device__ __forceinline__ void GatherTile(const PanelView& pv, int k0, int c0, 
     const int cq = (lane >> 4) * 4;
     const auto LU = dev::G(pv.src);
     const int tiles = (rows + 15) / 16;
-    dev::StaticFor<0, kMaxTiles>([&](auto tc) {
+    dev::StaticFor<0, N / 16>([&](auto tc) {
         constexpr int t = decltype(tc)::value;
         if (t < tiles) {
             const int row = 16 * t + r16;
@@ -409,8 +415,9 @@ __device__ __forceinline__ void GatherTile(const PanelView& pv, int k0, int c0, 
 }
 
 // The gathered tile: U12 = inv(L11) A12, update, store in position order.
-template <int P>
-__device__ __forceinline__ void UpdateTile(const PanelView& pv, int k0, int c0, FactorShared<P>& sh, SweepAcc& acc)
+template <int P, int N>
+__device__ __forceinline__ void UpdateTile(const PanelView& pv, int k0, int c0, FactorShared<P, N>& sh,
+                                           SweepAcc<N>& acc)
 {
     const int n = pv.n;
     const size_t ld = static_cast<size_t>(pv.ld);
@@ -473,7 +480,7 @@ __device__ __forceinline__ void UpdateTile(const PanelView& pv, int k0, int c0, 
             constexpr int st = decltype(sc)::value;
             ua[st] = sh.op.u[wave][r16][4 * st + grp];
         });
-        dev::StaticFor<2, kMaxTiles>([&](auto tc) {
+        dev::StaticFor<2, N / 16>([&](auto tc) {
             constexpr int t = decltype(tc)::value;
             if (t < tiles) {
                 const int lr = 16 * t - kNb + r16;
@@ -492,7 +499,7 @@ __device__ __forceinline__ void UpdateTile(const PanelView& pv, int k0, int c0, 
             constexpr int q = decltype(pc)::value;
             ub[q] = *reinterpret_cast<const bf16x8*>(&sh.op.u[wave][q][r16][kq]);
         });
-        dev::StaticFor<2, kMaxTiles>([&](auto tc) {
+        dev::StaticFor<2, N / 16>([&](auto tc) {
             constexpr int t = decltype(tc)::value;
             if (t < tiles) {
                 const int lr = 16 * t - kNb + r16;
@@ -519,7 +526,7 @@ __device__ __forceinline__ void UpdateTile(const PanelView& pv, int k0, int c0, 
         });
     }
 
-    dev::StaticFor<0, kMaxTiles>([&](auto tc) {
+    dev::StaticFor<0, N / 16>([&](auto tc) {
         constexpr int t = decltype(tc)::value;
         if (t < tiles) {
             const int row = 16 * t + r16;
@@ -539,14 +546,14 @@ __device__ __forceinline__ void UpdateTile(const PanelView& pv, int k0, int c0, 
 
 // The trailing columns k0 + width .. n-1 of the panel at k0, in 16-column
 // tiles dealt to the waves in turn.
-template <int P>
-__device__ __forceinline__ void SweepTrailing(const PanelView& pv, int k0, FactorShared<P>& sh)
+template <int P, int N>
+__device__ __forceinline__ void SweepTrailing(const PanelView& pv, int k0, FactorShared<P, N>& sh)
 {
     const int wave = static_cast<int>(threadIdx.x) / kWave;
     for (int c0 = k0 + kNb + wave * kTileN; c0 < pv.n; c0 += kWaves * kTileN) {
-        SweepAcc acc;
-        GatherTile<P>(pv, k0, c0, sh, acc);
-        UpdateTile<P>(pv, k0, c0, sh, acc);
+        SweepAcc<N> acc;
+        GatherTile<P, N>(pv, k0, c0, sh, acc);
+        UpdateTile<P, N>(pv, k0, c0, sh, acc);
     }
 }
 

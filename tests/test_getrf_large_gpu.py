@@ -100,3 +100,26 @@ def test_large_lu_ties_and_nan(handle):
     A[0, 5, 17] = np.nan
     A[1, 100, 100:] = np.nan
     _check(A, _getrf(handle, A))
+
+
+@pytest.mark.parametrize("n,batch", [(66, 1030), (127, 3), (128, 1025), (192, 3), (192, 770), (193, 515)])
+def test_blocked_lu_instances(handle, n, batch):
+    """64 < n <= 256: the instances of the blocked kernel (largest order 128, 192, 256) at their edges, with batches
+    past the persistent grid of each.  Pivots as the oracle's, P A = L U to the multiply-adds' rounding."""
+    A = _random(n, batch, shift=float(n) ** 0.5)
+    LU, piv, info = _getrf(handle, A)
+    assert not info.any()
+    some = np.unique(np.linspace(0, batch - 1, 9).astype(int))
+    _, gpiv, _ = O.getrf_batched(A[some].copy())
+    assert np.array_equal(piv[some], gpiv)
+    gamma = (n + 2) * 2.0 ** -24
+    for b in some:
+        M = LU[b].T.astype(np.float64)
+        L, U = np.tril(M, -1) + np.eye(n), np.triu(M)
+        P = A[b].T.astype(np.float64)
+        for k in range(n):
+            P[[k, piv[b, k] - 1]] = P[[piv[b, k] - 1, k]]
+        # U12 = inv(L11) A12 with an explicit inverse: its rounding is of the same order with |inv(L11)| |L11| terms
+        Li = np.abs(np.linalg.inv(L))
+        bound = 4 * gamma * (np.abs(L) @ Li @ np.abs(L) @ np.abs(U))
+        assert (np.abs(P - L @ U) <= bound).all()

@@ -112,26 +112,6 @@ __device__ __forceinline__ void BuildPerm(uint16_t* perm, uint16_t* from, const 
     Sync<WAVES>();
 }
 
-// x / u with r = 1 / u (correctly rounded): two residual corrections of x r.
-// The first leaves the quotient within one ulp, from where one more with the
-// rounded reciprocal gives the correctly rounded quotient (Markstein, IBM J.
-// Res. Dev. 34, 1990) while no intermediate under- or overflows: Dividable.
-__device__ __forceinline__ float DivideBy(float x, float u, float r)
-{
-    float q = x * r;
-    q = fmaf(fmaf(-u, q, x), r, q);
-    return fmaf(fmaf(-u, q, x), r, q);
-}
-
-// |v| in [2^-60, 2^60) (or +0 when ZERO): DivideBy is exact on such operands.
-template <bool ZERO>
-__device__ __forceinline__ bool Dividable(float v)
-{
-    const uint32_t u = __float_as_uint(v);
-    const bool range = (u & 0x7FFFFFFFu) - ((127u - 60u) << 23) < (120u << 23);
-    return range || (ZERO && u == 0u);
-}
-
 // The steps of a 16 x 16 diagonal block d ([column][row], in LDS) on the tile
 // y (accumulator layout: lane l holds rows 4 (l / 16) + j of right-hand side
 // l % 16), straight-line.  LOWER: k ascending, else descending.  The columns
@@ -166,8 +146,8 @@ __device__ __forceinline__ bool DiagSteps(float (&y)[4], const float (*d)[kT + 4
         if constexpr (!UNIT) {
             // meaningful in group g, which holds row k
             if constexpr (FAST) {
-                off = off || (grp == g && !Dividable<true>(v));
-                v = DivideBy(v, u[e], r[e]);
+                off = off || (grp == g && !dev::Dividable<true>(v));
+                v = dev::DivideBy(v, u[e], r[e]);
             } else {
                 v = v / u[e];
             }
@@ -204,7 +184,7 @@ __device__ __forceinline__ void SolveDiag(f32x4& x, const float (*d)[kT + 4], in
             constexpr int j = decltype(jc)::value;
             u[j] = d[4 * grp + j][4 * grp + j];
             r[j] = 1.0f / u[j];
-            off = off || (4 * grp + j < rows && !Dividable<false>(u[j]));
+            off = off || (4 * grp + j < rows && !dev::Dividable<false>(u[j]));
         });
         off = DiagSteps<LOWER, false, true>(y, d, u, r, rows, grp) || off;
         if (__builtin_amdgcn_ballot_w64(off) != 0) {

@@ -201,3 +201,48 @@ def test_mixed_solve_exact_ties(handle, update):
     assert (info == 0).all() and not fb.any()
     for s, x in zip(systems, xs):
         assert np.array_equal(x, s["X"]), (s["n"], np.abs(x - s["X"]).max())
+
+
+def _random_system(rng, n, r):
+    A = (rng.standard_normal((n, n)) + n * np.eye(n) * 0.25).astype(np.float32)
+    return {"n": n, "nrhs": r, "A": A.reshape(-1), "B": rng.standard_normal(n * r).astype(np.float32)}
+
+
+def _same_bits(a, b):
+    return all(np.array_equal(np.asarray(x).view(np.uint32), np.asarray(y).view(np.uint32)) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("update", ["FP32", "BF16", "BF16X2"])
+def test_mixed_solve_small_orders_apart(handle, update):
+    """Enough systems on both sides of order 128 that each side has its own launch: every copy of a system has the
+    bits that the system has in a call of a few (the instances differ in what they hold, not in the arithmetic)."""
+    rng = np.random.default_rng(29)
+    few = [_random_system(rng, n, r) for n, r in ((1, 1), (31, 16), (33, 3), (97, 9), (127, 8), (128, 16), (129, 5),
+                                                  (130, 16), (145, 1))]
+    want = _run(handle, few, 1e-7, 10, update)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    small = [i for i in range(len(few)) if few[i]["n"] <= 128]
+    large = [i for i in range(len(few)) if few[i]["n"] > 128]
+    for reps_small, reps_large in ((3 * cus // len(small) + 1, 3 * cus // len(large) + 1),
+                                   (3 * cus // len(small) + 1, 0)):
+        which = (small * reps_small + large * reps_large)
+        rng.shuffle(which)
+        got = _run(handle, [few[i] for i in which], 1e-7, 10, update)
+        assert _same_bits(got[0], [want[0][i] for i in which])
+        for k in range(1, 5):
+            assert np.array_equal(got[k], want[k][which]), k
+
+
+@pytest.mark.parametrize("exponent", [-62, 70])
+def test_mixed_solve_divisors_out_of_range(handle, exponent):
+    """Scaling A and B by a power of two scales U and leaves everything else as it is, bit for bit; at these scales
+    the substitution's quotients leave the range of the shared reciprocals and are divided one by one."""
+    rng = np.random.default_rng(31)
+    systems = [_random_system(rng, n, r) for n, r in ((32, 16), (64, 5), (100, 12), (256, 16))]
+    scaled = [dict(s, A=s["A"] * np.float32(2.0 ** exponent), B=s["B"] * np.float32(2.0 ** exponent)) for s in systems]
+    for update in ("FP32", "BF16X2"):
+        want = _run(handle, systems, 1e-6, 10, update)
+        got = _run(handle, scaled, 1e-6, 10, update)
+        assert _same_bits(got[0], want[0])
+        for k in range(1, 5):
+            assert np.array_equal(got[k], want[k]), k

@@ -71,6 +71,28 @@ def test_quantizer_unaligned_operands(handle, xoff, qoff):
     assert not got[:qoff].any()
 
 
+@pytest.mark.parametrize("qt", ["FP8_E4M3FN", "FP8_E5M2"])
+@pytest.mark.parametrize("count", [(1 << 22) - 4, 1 << 22, (1 << 22) + 4, 5 * (1 << 20) + 7])
+def test_quantizer_rounding_points(handle, qt, count):
+    """With amax = fp8_max (scale 1): every value of the format, every midpoint between neighbours and the FP32 numbers
+    next to it, both signs, in a tensor around four whole steps of the grid; a NaN keeps its sign and takes its three
+    neighbours through the other conversion."""
+    e4m3 = qt == "FP8_E4M3FN"
+    dt = torch.float8_e4m3fn if e4m3 else torch.float8_e5m2
+    v = torch.arange(0x7F if e4m3 else 0x7C, dtype=torch.uint8).view(dt).float().numpy()
+    mid = (v[:-1] + v[1:]) / np.float32(2)
+    pts = np.concatenate([v, mid, np.nextafter(mid, np.float32(0)), np.nextafter(mid, np.float32(1e9))])
+    pts = np.concatenate([pts, -pts, [1e-39, -1e-45]]).astype(np.float32)
+    x = np.resize(pts, count)
+    x[-1] = FMAX[qt]
+    ref = O.to_fp8(x, e4m3)
+    x[1001], x[count // 2] = np.float32(np.nan), np.copysign(np.float32(np.nan), np.float32(-1))
+    ref[1001], ref[count // 2] = 0x7F, 0xFF
+    q, s, _, _ = _quantize(handle, x, qt)
+    assert s == 1.0
+    assert np.array_equal(q, ref), int((q != ref).sum())
+
+
 def test_quantizer_all_zero(handle):
     q, s, _, _ = _quantize(handle, np.zeros(4097, np.float32), "FP8_E4M3FN")
     assert s == 1.0 and not q.any()

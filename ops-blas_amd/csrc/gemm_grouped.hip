@@ -1,6 +1,7 @@
 // aclblasSgemmGroupedBatched: FP32 GEMMs of several shapes in one launch;
 // aclblasGemmGroupedBatchedEx (FP16 / BF16 / FP8, device pointer arrays) at the
-// end of the file, on the same persistent kernel.
+// end of the file, on the same persistent kernel or, for 16-bit problems that
+// qualify, on the direct-to-LDS tile.
 //
 // Reference: blas/gemm_grouped_batched/arch35/gemm_grouped_batched_host.cpp
 // (argument checks :155-290 and :448-477 in that order; inactive groups

@@ -38,7 +38,7 @@
 // What bounds it: the LDS round trips at the start of a stage (its fragments
 // can only be read after the barrier) against 32 matrix instructions per wave
 // with 256 x 256 tiles and 16 with 128 x 128; the larger tile, whose two waves
-// per SIMD also cover for each other, reaches 1.4 PFLOP/s.  4096^3, BF16 out, A
+// per SIMD also cover for each other, reaches 1.6 PFLOP/s.  4096^3, BF16 out, A
 // and B K-contiguous (NT) / both row-contiguous (TN): MXFP8 332 -> 84 / 2490
 // -> 88 us, MXFP4 191 -> 76 / 1523 -> 62 us (before: 64 x 64 tiles, element-wise
 // transposes, no load in flight during the products).  Fragments of the next

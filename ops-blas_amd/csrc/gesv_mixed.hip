@@ -101,7 +101,7 @@ struct MixedSystem {
 __device__ __forceinline__ int RowMapOffset(int n, int p) { return p * n - 16 * p * (p - 1); }
 
 template <int P, int N>
-__global__ __launch_bounds__(kThreads, N == kMaxN ? 3 : 4) void GesvFactorKernel(const MixedSystem* __restrict__ systems,
+__global__ __launch_bounds__(kThreads, N > 128 ? 3 : 4) void GesvFactorKernel(const MixedSystem* __restrict__ systems,
                                                                                  int count, int onlyMarked)
 {
     __shared__ __attribute__((aligned(16))) FactorShared<P, N> sh;
@@ -248,7 +248,7 @@ template <int N>
 __device__ __forceinline__ void FactoredSolve(const MixedSystem& s, RefineShared<N>& sh)
 {
     constexpr int kWaves = N / kWave;
-    constexpr int kOwn = (N / 16 - 2 + kWaves - 1) / kWaves;  // 16-row blocks of a wave: 4 or 3
+    constexpr int kOwn = (N / 16 - 2 + kWaves - 1) / kWaves;  // 16-row blocks of a wave: 4, or 3 for N = 128
     constexpr int kRhsWave = kMaxRhs / kWaves;
     const int n = s.n;
     const int t = threadIdx.x;
@@ -767,8 +767,8 @@ namespace aclblas {
 namespace {
 
 constexpr size_t kAlign = 256;
-constexpr int kSmallN = 128;   // largest order of the smaller instances
-constexpr int kFillPerCu = 3;  // systems per CU from which a part has a launch of its own
+constexpr int kSmallN = 128;  // largest orders of the smaller instances
+constexpr int kMidN = 192;
 
 size_t AlignUp(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 
@@ -817,23 +817,34 @@ aclblasStatus_t ValidateMixed(int batch, const int* nA, const int* rA, const flo
     return ACLBLAS_STATUS_SUCCESS;
 }
 
+// Systems first .. last - 1 of the table.
 template <int N>
-void LaunchFactor(int update, int perCu, int cus, hipStream_t stream, const MixedSystem* sys, int count, int onlyMarked)
+void LaunchFactor(int update, int perCu, int cus, hipStream_t stream, const MixedSystem* table, int first, int last,
+                  int onlyMarked)
 {
+    const int count = last - first;
+    const MixedSystem* sys = table + first;
+    if (count <= 0) {
+        return;
+    }
     const dim3 grid(static_cast<unsigned>(std::min(count, perCu * cus)));
-    switch (update) {
-    case ACLBLAS_MIXED_UPDATE_BF16:
-        hipLaunchKernelGGL((GesvFactorKernel<1, N>), grid, dim3(kThreads), 0, stream, sys, count, onlyMarked);
-        break;
-    case ACLBLAS_MIXED_UPDATE_BF16X2:
-        hipLaunchKernelGGL((GesvFactorKernel<2, N>), grid, dim3(kThreads), 0, stream, sys, count, onlyMarked);
-        break;
-    case ACLBLAS_MIXED_UPDATE_BF16X3:
-        hipLaunchKernelGGL((GesvFactorKernel<3, N>), grid, dim3(kThreads), 0, stream, sys, count, onlyMarked);
-        break;
-    default:
+    if constexpr (N < kMaxN) {  // FP32 updates only
         hipLaunchKernelGGL((GesvFactorKernel<0, N>), grid, dim3(kThreads), 0, stream, sys, count, onlyMarked);
-        break;
+    } else {
+        switch (update) {
+        case ACLBLAS_MIXED_UPDATE_BF16:
+            hipLaunchKernelGGL((GesvFactorKernel<1, N>), grid, dim3(kThreads), 0, stream, sys, count, onlyMarked);
+            break;
+        case ACLBLAS_MIXED_UPDATE_BF16X2:
+            hipLaunchKernelGGL((GesvFactorKernel<2, N>), grid, dim3(kThreads), 0, stream, sys, count, onlyMarked);
+            break;
+        case ACLBLAS_MIXED_UPDATE_BF16X3:
+            hipLaunchKernelGGL((GesvFactorKernel<3, N>), grid, dim3(kThreads), 0, stream, sys, count, onlyMarked);
+            break;
+        default:
+            hipLaunchKernelGGL((GesvFactorKernel<0, N>), grid, dim3(kThreads), 0, stream, sys, count, onlyMarked);
+            break;
+        }
     }
 }
 
@@ -924,47 +935,55 @@ extern "C" aclblasStatus_t aclblasSgesvBatchedMixedEx(
     const MixedSystem* sys = static_cast<const MixedSystem*>(dev);
     hipStream_t stream = handle->stream;
     const int mayMark = mode != ACLBLAS_MIXED_UPDATE_FP32 ? 1 : 0;
-    // Orders up to kSmallN on the kernels' smaller instances, where more systems
-    // share a CU (factor four for three, solve six two-wave workgroups for three
-    // of four waves, whose upper two have no rows there): 10000 systems of order
-    // 16..256 in 4.93 ms for 5.10 in single launches.  Only when each part fills
-    // the card; below that a second launch would wait for the first one's last
-    // systems, and one launch runs all of them side by side.
-    const int large = static_cast<int>(
-        std::partition_point(table.begin(), table.end(), [](const MixedSystem& s) { return s.n > kSmallN; }) -
-        table.begin());
-    const int small = batchCount - large;
-    const bool split = small >= kFillPerCu * cus && (large == 0 || large >= kFillPerCu * cus);
-    const int first = split ? large : batchCount;
+    // Smaller instances, of which more fit a CU, in launches of their own: the
+    // solve up to kSmallN (six two-wave workgroups per CU for three of four
+    // waves, whose upper two have no rows there) and, with FP32 updates, the
+    // factorisation up to kSmallN and kMidN (four and three workgroups per CU
+    // for two; the BF16 instances are at three already and gained nothing from a
+    // fourth).  Only when each part fills the card several times: the next
+    // launch waits for the last systems of the one before.  Orders 16..256, us
+    // per call in one launch per stage / in parts: BF16X2 10000 systems 5102 /
+    // 5022, 2800 1710 / 1674, 2200 1327 / 1384 (so not split); FP32 8000 systems
+    // 3900 / 3670, 3300 1901 / 1711, 2500 1423 / 1472 (not split).
+    const auto above = [&](int n) {
+        return static_cast<int>(
+            std::partition_point(table.begin(), table.end(), [n](const MixedSystem& s) { return s.n > n; }) -
+            table.begin());
+    };
+    const auto fills = [&](int first, int last, int perCu) { return last - first >= perCu * cus; };
+    const int n128 = above(kSmallN);
+    const int n192 = above(kMidN);
+    const bool split = fills(n128, batchCount, 5) && (n128 == 0 || fills(0, n128, 5));
+    const int smallFrom = split ? n128 : batchCount;
     MarkLaunch(handle, 0);
-    if (first > 0) {
-        LaunchFactor<kMaxN>(mode, c.a, cus, stream, sys, first, 0);
-    }
-    if (split) {
-        LaunchFactor<kSmallN>(mode, c.a + 1, cus, stream, sys + first, small, 0);
+    if (split && mode == ACLBLAS_MIXED_UPDATE_FP32) {
+        const int midFrom = fills(n192, n128, 3) && (n192 == 0 || fills(0, n192, 3)) ? n192 : n128;
+        LaunchFactor<kMaxN>(mode, c.a, cus, stream, sys, 0, midFrom, 0);
+        LaunchFactor<kMidN>(mode, c.a + 1, cus, stream, sys, midFrom, n128, 0);
+        LaunchFactor<kSmallN>(mode, c.a + 2, cus, stream, sys, n128, batchCount, 0);
+    } else {
+        LaunchFactor<kMaxN>(mode, c.a, cus, stream, sys, 0, batchCount, 0);
     }
     MarkLaunch(handle, 1);
     MarkLaunch(handle, 2);
-    if (first > 0) {
-        hipLaunchKernelGGL(GesvRefineKernel<kMaxN>, dim3(static_cast<unsigned>(std::min(first, c.b * cus))),
-                           dim3(kMaxN), 0, stream, sys, first, tol, maxIter, mayMark, 0, iterArray, berrArray,
-                           infoArray, fallbackArray);
-    }
-    if (split) {
-        hipLaunchKernelGGL(GesvRefineKernel<kSmallN>,
-                           dim3(static_cast<unsigned>(std::min(small, kMaxN / kSmallN * c.b * cus))), dim3(kSmallN), 0,
-                           stream, sys + first, small, tol, maxIter, mayMark, 0, iterArray, berrArray, infoArray,
-                           fallbackArray);
-    }
+    const auto refine = [&](auto nc, int first, int last, int mark, int onlyMarked) {
+        constexpr int N = decltype(nc)::value;
+        if (first < last) {
+            hipLaunchKernelGGL(GesvRefineKernel<N>,
+                               dim3(static_cast<unsigned>(std::min(last - first, kMaxN * c.b / N * cus))), dim3(N), 0,
+                               stream, sys + first, last - first, tol, maxIter, mark, onlyMarked, iterArray, berrArray,
+                               infoArray, fallbackArray);
+        }
+    };
+    refine(std::integral_constant<int, kMaxN>{}, 0, smallFrom, mayMark, 0);
+    refine(std::integral_constant<int, kSmallN>{}, smallFrom, batchCount, mayMark, 0);
     MarkLaunch(handle, 3);
     if (mayMark != 0) {
         MarkLaunch(handle, 4);
-        LaunchFactor<kMaxN>(ACLBLAS_MIXED_UPDATE_FP32, c.a, cus, stream, sys, batchCount, 1);
+        LaunchFactor<kMaxN>(ACLBLAS_MIXED_UPDATE_FP32, c.a, cus, stream, sys, 0, batchCount, 1);
         MarkLaunch(handle, 5);
         MarkLaunch(handle, 6);
-        hipLaunchKernelGGL(GesvRefineKernel<kMaxN>, dim3(static_cast<unsigned>(std::min(batchCount, c.b * cus))),
-                           dim3(kMaxN), 0, stream, sys, batchCount, tol, maxIter, 0, 1, iterArray, berrArray, infoArray,
-                           fallbackArray);
+        refine(std::integral_constant<int, kMaxN>{}, 0, batchCount, 0, 1);
         MarkLaunch(handle, 7);
     }
     return LaunchStatus("aclblasSgesvBatchedMixedEx");

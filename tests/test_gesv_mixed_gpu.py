@@ -214,18 +214,18 @@ def _same_bits(a, b):
 
 @pytest.mark.parametrize("update", ["FP32", "BF16", "BF16X2"])
 def test_mixed_solve_small_orders_apart(handle, update):
-    """Enough systems on both sides of order 128 that each side has its own launch: every copy of a system has the
-    bits that the system has in a call of a few (the instances differ in what they hold, not in the arithmetic)."""
+    """Enough systems up to order 128, from there to 192 and above that each part has its own launch: every copy of a
+    system has the bits that the system has in a call of a few (the instances differ in what they hold, not in the
+    arithmetic)."""
     rng = np.random.default_rng(29)
     few = [_random_system(rng, n, r) for n, r in ((1, 1), (31, 16), (33, 3), (97, 9), (127, 8), (128, 16), (129, 5),
-                                                  (130, 16), (145, 1))]
+                                                  (130, 16), (145, 1), (191, 7), (192, 16), (193, 16), (225, 4))]
     want = _run(handle, few, 1e-7, 10, update)
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
-    small = [i for i in range(len(few)) if few[i]["n"] <= 128]
-    large = [i for i in range(len(few)) if few[i]["n"] > 128]
-    for reps_small, reps_large in ((3 * cus // len(small) + 1, 3 * cus // len(large) + 1),
-                                   (3 * cus // len(small) + 1, 0)):
-        which = (small * reps_small + large * reps_large)
+    need = 5 * torch.cuda.get_device_properties(0).multi_processor_count
+    parts = [[i for i in range(len(few)) if lo < few[i]["n"] <= hi] for lo, hi in ((0, 128), (128, 192), (192, 256))]
+    for counts in ((need, need, need), (need, need, 0), (need, 0, need), (need, 0, 0), (need, need - 9, 9),
+                   (need - 1, need, 9)):
+        which = [i for part, count in zip(parts, counts) for i in (part * (count // len(part) + 1))[:count]]
         rng.shuffle(which)
         got = _run(handle, [few[i] for i in which], 1e-7, 10, update)
         assert _same_bits(got[0], [want[0][i] for i in which])

@@ -673,6 +673,18 @@ __global__ __launch_bounds__(N, 3) void GesvRefineKernel(const MixedSystem* __re
             }
             continue;
         }
+        if (n == 0 || nrhs == 0) {
+            // nothing to solve, and nothing to read: no panel, inverse or row map
+            // exists for order 0, and B may be null
+            if (t == 0) {
+                if (iterOut != nullptr) iterOut[s.index] = 0;
+                if (berrOut != nullptr) berrOut[s.index] = 0.0f;
+                if (infoOut != nullptr) infoOut[s.index] = 0;
+                if (fallbackOut != nullptr) fallbackOut[s.index] = onlyMarked;
+                dev::G(s.state)[1] = 0;
+            }
+            continue;
+        }
         // x0 = LU \ b (rows >= n and columns >= nrhs of bs and x are zero)
         {
             float b0[kMaxRhs];

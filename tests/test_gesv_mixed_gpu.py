@@ -246,3 +246,50 @@ def test_mixed_solve_divisors_out_of_range(handle, exponent):
         assert _same_bits(got[0], want[0])
         for k in range(1, 5):
             assert np.array_equal(got[k], want[k]), k
+
+
+@pytest.mark.parametrize("update", ["FP32", "BF16", "BF16X2", "BF16X3"])
+@pytest.mark.parametrize("copies", [1, 40])
+def test_mixed_solve_empty_members(handle, update, copies):
+    """Members of order 0 and members without right-hand sides (null pointers where there is nothing to point at) among
+    ordinary ones, in a few systems (one launch per stage) and in enough for the launches by order: they report 0
+    corrections, backward error 0 and info 0, a singular matrix its column; the others solve as without them."""
+    rng = np.random.default_rng(31)
+    ordinary = [_random_system(rng, n, r) for n, r in ((1, 1), (33, 3), (128, 16), (129, 5), (256, 2))] * copies
+    if copies > 1:
+        need = 5 * torch.cuda.get_device_properties(0).multi_processor_count
+        ordinary += [_random_system(rng, n, 1) for n in (5, 130) for _ in range(need)]
+    singular = _random_system(rng, 20, 0)
+    singular["A"][40:60] = 0.0                       # column 2
+    empty = [_random_system(rng, n, r) for n, r in ((0, 0), (0, 3), (0, 16), (1, 0), (32, 0), (130, 0), (256, 0))]
+    want = _run(handle, ordinary, 1e-6, 10, update)
+    systems = ordinary + (empty + [singular]) * copies
+    dA, dB, dX, pa, pb, px, offB = _upload(systems)
+    ns, rs = [s["n"] for s in systems], [s["nrhs"] for s in systems]
+    pa = [p if n else 0 for p, n in zip(pa, ns)]
+    pb = [p if n * r else 0 for p, n, r in zip(pb, ns, rs)]
+    px = [p if n * r else 0 for p, n, r in zip(px, ns, rs)]
+    ld = [max(1, n) for n in ns]
+    out = [torch.full((len(systems),), -1, dtype=t, device="cuda")
+           for t in (torch.int32, torch.float32, torch.int32, torch.int32)]
+    assert B.sgesv_batched_mixed_ex(handle.value, ns, rs, pa, ld, pb, ld, px, ld, 1e-6, 10, B.MIXED_UPDATE[update],
+                                    *[t.data_ptr() for t in out]) == 0
+    torch.cuda.synchronize()
+    iters, berr, info, fb = [t.cpu().numpy() for t in out]
+    k = len(ordinary)
+    X = dX.cpu().numpy()
+    if update != "BF16X3":   # three planes are not reproducible from call to call
+        assert _same_bits([X[o:o + s["n"] * s["nrhs"]] for o, s in zip(offB, ordinary)], want[0])
+    else:
+        _check_backward(ordinary, [X[o:o + s["n"] * s["nrhs"]] for o, s in zip(offB, ordinary)], 1e-6)
+    assert (info[:k] == 0).all() and (berr[:k] <= 1e-6).all()
+    sing = np.array([s is singular for s in systems[k:]])
+    assert (iters[k:] == 0).all()
+    assert (info[k:][~sing] == 0).all() and (info[k:][sing] == 3).all(), info[k:]
+    assert (berr[k:][~sing] == 0).all() and np.isinf(berr[k:][sing]).all()
+    assert (fb[k:][~sing] == 0).all() and (fb[k:][sing] == (0 if update == "FP32" else 1)).all()
+
+
+def _check_backward(systems, xs, tol):
+    for s, x in zip(systems, xs):
+        assert W.normwise_backward_error(s["A"], s["n"], s["B"], x, s["nrhs"]) <= tol, (s["n"], s["nrhs"])

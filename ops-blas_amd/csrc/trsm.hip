@@ -277,7 +277,7 @@ __global__ __launch_bounds__(kDiagThreads) void TrsmInnerKernel(DiagArgs p)
 }
 
 // inner: ascending inner products instead of the backward column sweep.
-void LaunchDiag(hipStream_t st, bool left, const DiagArgs& p, bool forward, bool inner)
+void LaunchSlice(hipStream_t st, bool left, const DiagArgs& p, bool forward, bool inner)
 {
     if (inner) {
         const dim3 grid(static_cast<unsigned>((p.vectors + kDiagThreads - 1) / kDiagThreads));
@@ -302,6 +302,19 @@ void LaunchDiag(hipStream_t st, bool left, const DiagArgs& p, bool forward, bool
         } else {
             hipLaunchKernelGGL((TrsmSweepKernel<false, false>), grid, block, 0, st, p);
         }
+    }
+}
+
+// A launch has fewer than 2^32 threads, and the sweep takes up to 32 a vector:
+// at most kSlice vectors (2^31 threads) each.
+void LaunchDiag(hipStream_t st, bool left, const DiagArgs& p, bool forward, bool inner)
+{
+    constexpr long long kSlice = 1ll << 26;
+    for (long long v0 = 0; v0 < p.vectors; v0 += kSlice) {
+        DiagArgs q = p;
+        q.B = p.B + (left ? v0 * p.ldb : v0);
+        q.vectors = static_cast<int>(p.vectors - v0 < kSlice ? p.vectors - v0 : kSlice);
+        LaunchSlice(st, left, q, forward, inner);
     }
 }
 

@@ -192,3 +192,27 @@ def test_strsm_one_block_bitwise(handle, dim, side, uplo, trans, diag):
     st, out = _call(handle, row, a, b)
     assert st == 0
     assert np.array_equal(out[:(m + 2) * n], _gold(row, a, b)[:(m + 2) * n])
+
+
+@pytest.mark.parametrize("dim", [1, 33])
+@pytest.mark.parametrize("side", ["LEFT", "RIGHT"])
+def test_strsm_more_vectors_than_a_launch_holds(handle, dim, side):
+    """2^27 + 5 right-hand-side vectors, with up to 32 threads each: more than the 2^32 threads of one launch.
+    M = 2 I + ones below the first diagonal entry, B = 1: y = (1/2, 1/4, 1/4, ...) exactly."""
+    count = (1 << 27) + 5
+    left = side == "LEFT"
+    # columns of A; the right side solves with A^T's lower triangle, so A is upper there
+    M = 2 * torch.eye(dim, device="cuda")
+    M[1:, 0] = 1.0                                   # row i, column 0 of the lower factor
+    a = (M.T if left else M).contiguous()            # column-major storage of M, or of M^T
+    x = torch.ones((count, dim) if left else (dim, count), dtype=torch.float32, device="cuda")
+    m, n = (dim, count) if left else (count, dim)
+    st = B.strsm(handle.value, B.SIDE[side], B.FILL["LOWER" if left else "UPPER"], B.OP_N, B.DIAG["NON_UNIT"], m, n,
+                 1.0, a.data_ptr(), dim, x.data_ptr(), m)
+    assert st == 0, st
+    y = x if left else x.T
+    assert bool((y[:, 0] == 0.5).all())
+    for i in range(1, dim):
+        assert bool((y[:, i] == 0.25).all()), i
+    del x, y
+    torch.cuda.empty_cache()

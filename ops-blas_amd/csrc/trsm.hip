@@ -32,8 +32,6 @@ namespace {
 
 constexpr int kTb = 128;         // diagonal block order
 constexpr int kVec = 16;         // tile order, and vectors per workgroup of the sweep kernel
-constexpr int kSweepThreads = kTb / kVec * 64;  // one wave per tile of the block
-constexpr int kBlockLoads = kTb * kTb / kSweepThreads;
 constexpr int kDiagThreads = 64;  // vectors per workgroup of the inner-product kernel
 
 // B[i + j ldb] *= alpha (or = 0 when zero), i < m, j < n.
@@ -81,8 +79,8 @@ __device__ __forceinline__ size_t BOffset(const DiagArgs& p, int i, int vec)
 }
 
 // Column sweeps (forward: k ascending, else descending; each finished y_k is
-// subtracted from the rows still open), 16 vectors per workgroup of eight
-// waves.  Wave I holds rows 16 I .. 16 I + 15 as one tile (dev::F32x4 layout);
+// subtracted from the rows still open), 16 vectors per workgroup of NT waves
+// (eight for a whole block).  Wave I holds rows 16 I .. 16 I + 15 as one tile (dev::F32x4 layout);
 // in phase J wave J solves its 16 x 16 block and publishes y, then the waves
 // behind it subtract the block's 16 columns in k order, wave J + 1 first of
 // all finishing its tile.  The block lies in LDS as [column][row], so a wave
@@ -92,10 +90,13 @@ __device__ __forceinline__ size_t BOffset(const DiagArgs& p, int i, int vec)
 // lane per vector with its values in LDS (before) took 255 us for a block of
 // 128 and 1000 vectors: 16 waves on the GPU, one dependent LDS round trip per
 // multiply-subtract; this takes 19 us (504 waves).
-template <bool LEFT, bool FORWARD>
-__global__ __launch_bounds__(kSweepThreads) void TrsmSweepKernel(DiagArgs p)
+template <bool LEFT, bool FORWARD, int NT>
+__global__ __launch_bounds__(NT * dev::kWave) void TrsmSweepKernel(DiagArgs p)
 {
-    __shared__ __attribute__((aligned(16))) float T[kTb][kTb + 4];  // [column][row]
+    constexpr int kN = NT * kVec;
+    constexpr int kThreads = NT * dev::kWave;
+    constexpr int kBlockLoads = kN * kN / kThreads;
+    __shared__ __attribute__((aligned(16))) float T[kN][kN + 4];    // [column][row]
     __shared__ float ys[2][kVec][kVec];                             // y of the solved block, [k][vector]
     const int tid = threadIdx.x;
     const int lane = dev::LaneId();
@@ -116,8 +117,8 @@ __global__ __launch_bounds__(kSweepThreads) void TrsmSweepKernel(DiagArgs p)
     float m[kBlockLoads];
     dev::StaticFor<0, kBlockLoads>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
-        const int fast = min(tid % kTb, p.kb - 1);
-        const int slow = min(tid / kTb + q * (kSweepThreads / kTb), p.kb - 1);
+        const int fast = min(tid % kN, p.kb - 1);
+        const int slow = min(tid / kN + q * (kThreads / kN), p.kb - 1);
         m[q] = p.readDirect != 0 ? LoadM(p, fast, slow) : LoadM(p, slow, fast);
     });
     dev::StaticFor<0, 4>([&](auto jc) {
@@ -126,8 +127,8 @@ __global__ __launch_bounds__(kSweepThreads) void TrsmSweepKernel(DiagArgs p)
     });
     dev::StaticFor<0, kBlockLoads>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
-        const int fast = tid % kTb;
-        const int slow = tid / kTb + q * (kSweepThreads / kTb);
+        const int fast = tid % kN;
+        const int slow = tid / kN + q * (kThreads / kN);
         const int i = p.readDirect != 0 ? fast : slow;
         const int j = p.readDirect != 0 ? slow : fast;
         const bool in = i < p.kb && j < p.kb && (i == j ? p.unit == 0 : (FORWARD ? i > j : i < j));
@@ -192,23 +193,27 @@ __global__ __launch_bounds__(kSweepThreads) void TrsmSweepKernel(DiagArgs p)
 // solved last and the whole block is one chain of kb^2 / 2 subtractions: one
 // lane per vector, the vectors' values in LDS columns.  128 x 1000: 210 us
 // with an LDS round trip per product, 159 us.
-template <bool LEFT>
+template <bool LEFT, int NT>
 __global__ __launch_bounds__(kDiagThreads) void TrsmInnerKernel(DiagArgs p)
 {
-    __shared__ __attribute__((aligned(16))) float T[kTb][kTb];  // [row][column]
-    __shared__ float ys[kTb][kDiagThreads];
+    constexpr int kN = NT * kVec;
+    constexpr int kRowLoads = (kN + kDiagThreads - 1) / kDiagThreads;
+    __shared__ __attribute__((aligned(16))) float T[kN][kN];  // [row][column]
+    __shared__ float ys[kN][kDiagThreads];
     const int tid = threadIdx.x;
 #pragma unroll 8
     for (int i = 0; i < p.kb; ++i) {
-        float m[kTb / kDiagThreads];
+        float m[kRowLoads];
 #pragma unroll
-        for (int q = 0; q < kTb / kDiagThreads; ++q) {
+        for (int q = 0; q < kRowLoads; ++q) {
             m[q] = LoadM(p, i, min(tid + q * kDiagThreads, p.kb - 1));
         }
 #pragma unroll
-        for (int q = 0; q < kTb / kDiagThreads; ++q) {
+        for (int q = 0; q < kRowLoads; ++q) {
             const int j = tid + q * kDiagThreads;
-            T[i][j] = j < p.kb && (i == j ? p.unit == 0 : i < j) ? m[q] : (i == j ? 1.0f : 0.0f);
+            if (j < kN) {
+                T[i][j] = j < p.kb && (i == j ? p.unit == 0 : i < j) ? m[q] : (i == j ? 1.0f : 0.0f);
+            }
         }
     }
     const int vec = static_cast<int>(blockIdx.x) * kDiagThreads + tid;
@@ -218,8 +223,8 @@ __global__ __launch_bounds__(kDiagThreads) void TrsmInnerKernel(DiagArgs p)
         const float v = dev::G(p.B)[BOffset<LEFT>(p, i, min(vec, p.vectors - 1))];
         ys[i][tid] = valid ? v : 0.0f;
     }
-    for (int i = p.kb; i < kTb; ++i) {
-        ys[i][tid] = 0.0f;  // columns past kb: zero products
+    for (int i = p.kb; i < ((p.kb + 7) & ~7); ++i) {
+        ys[i][tid] = 0.0f;  // columns past kb, to a whole group of eight: zero products
     }
     __syncthreads();
     // eight products at a time, the next eight operands loaded before the
@@ -276,32 +281,47 @@ __global__ __launch_bounds__(kDiagThreads) void TrsmInnerKernel(DiagArgs p)
     }
 }
 
-// inner: ascending inner products instead of the backward column sweep.
-void LaunchSlice(hipStream_t st, bool left, const DiagArgs& p, bool forward, bool inner)
+// NT tiles: the block's order at most 16 NT.  inner: ascending inner products
+// instead of the backward column sweep.
+template <int NT>
+void LaunchTiles(hipStream_t st, bool left, const DiagArgs& p, bool forward, bool inner)
 {
+    const int per = inner ? kDiagThreads : kVec;
+    const dim3 grid(static_cast<unsigned>((p.vectors + per - 1) / per));
+    const dim3 block(inner ? kDiagThreads : NT * dev::kWave);
     if (inner) {
-        const dim3 grid(static_cast<unsigned>((p.vectors + kDiagThreads - 1) / kDiagThreads));
         if (left) {
-            hipLaunchKernelGGL(TrsmInnerKernel<true>, grid, dim3(kDiagThreads), 0, st, p);
+            hipLaunchKernelGGL((TrsmInnerKernel<true, NT>), grid, block, 0, st, p);
         } else {
-            hipLaunchKernelGGL(TrsmInnerKernel<false>, grid, dim3(kDiagThreads), 0, st, p);
+            hipLaunchKernelGGL((TrsmInnerKernel<false, NT>), grid, block, 0, st, p);
         }
-        return;
-    }
-    const dim3 grid(static_cast<unsigned>((p.vectors + kVec - 1) / kVec));
-    const dim3 block(kSweepThreads);
-    if (left) {
+    } else if (left) {
         if (forward) {
-            hipLaunchKernelGGL((TrsmSweepKernel<true, true>), grid, block, 0, st, p);
+            hipLaunchKernelGGL((TrsmSweepKernel<true, true, NT>), grid, block, 0, st, p);
         } else {
-            hipLaunchKernelGGL((TrsmSweepKernel<true, false>), grid, block, 0, st, p);
+            hipLaunchKernelGGL((TrsmSweepKernel<true, false, NT>), grid, block, 0, st, p);
         }
     } else {
         if (forward) {
-            hipLaunchKernelGGL((TrsmSweepKernel<false, true>), grid, block, 0, st, p);
+            hipLaunchKernelGGL((TrsmSweepKernel<false, true, NT>), grid, block, 0, st, p);
         } else {
-            hipLaunchKernelGGL((TrsmSweepKernel<false, false>), grid, block, 0, st, p);
+            hipLaunchKernelGGL((TrsmSweepKernel<false, false, NT>), grid, block, 0, st, p);
         }
+    }
+}
+
+// A small block on an instance of its size: with the LDS and the waves of a
+// block of 128 the sweep takes 611 us for order 4 and 10^6 vectors (45 us on
+// one wave a workgroup) and 132 us for order 16 and 200000 (13 us), the inner
+// products 279 and 120 us (13 and 13 us).
+void LaunchSlice(hipStream_t st, bool left, const DiagArgs& p, bool forward, bool inner)
+{
+    if (p.kb <= kVec) {
+        LaunchTiles<1>(st, left, p, forward, inner);
+    } else if (p.kb <= 2 * kVec) {
+        LaunchTiles<2>(st, left, p, forward, inner);
+    } else {
+        LaunchTiles<kTb / kVec>(st, left, p, forward, inner);
     }
 }
 

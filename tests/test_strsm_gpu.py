@@ -216,3 +216,13 @@ def test_strsm_more_vectors_than_a_launch_holds(handle, dim, side):
         assert bool((y[:, i] == 0.25).all()), i
     del x, y
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("dim", [5, 24, 31, 32, 33])
+@pytest.mark.parametrize("side", ["LEFT", "RIGHT"])
+@pytest.mark.parametrize("uplo", ["LOWER", "UPPER"])
+@pytest.mark.parametrize("trans", ["N", "T"])
+@pytest.mark.parametrize("diag", ["NON_UNIT", "UNIT"])
+def test_strsm_small_block_bitwise(handle, dim, side, uplo, trans, diag):
+    """Orders around those where the instances of one and two tiles end."""
+    test_strsm_one_block_bitwise(handle, dim, side, uplo, trans, diag)

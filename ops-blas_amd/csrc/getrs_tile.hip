@@ -606,13 +606,24 @@ void LaunchSolveTile(hipStream_t st, int n, int nrhs, const float* const* A, int
     // unit halves the latency and wastes issue slots on waiting waves.  Order
     // 128, 8 right-hand sides, N: 256 systems 47 (wave) and 34 us (workgroup),
     // 1024: 50 and 50, 2048: 66 and 96; order 250: 1024 systems 131 and 113.
-    // More than 16 tiles go to 16 waves.
-    if (n > 256) {
-        Launch<MODE, 16>(st, p, batch);
-    } else if (units >= 1536) {
-        Launch<MODE, 1>(st, p, batch);
-    } else {
+    // Past order 256 (more than 16 tiles) 16 waves have the lowest latency, and
+    // fewer of them more units on a CU, up to the orders of which only one fits
+    // it.  N, 1 right-hand side, us with 16 / 8 / 4 waves: order 257, 256 systems
+    // 64 / 67 / 74, 2000 systems 510 / 327 / 229; order 700, 256 systems 205 /
+    // 224 / 327, 1000 systems 823 / 615 / 772; order 1200, 300 systems 861 /
+    // 1063 / 1819.
+    if (n <= 256) {
+        if (units >= 1536) {
+            Launch<MODE, 1>(st, p, batch);
+        } else {
+            Launch<MODE, 4>(st, p, batch);
+        }
+    } else if (units > 256 && n <= 512) {
         Launch<MODE, 4>(st, p, batch);
+    } else if (units > 256 && n <= 1024) {
+        Launch<MODE, 8>(st, p, batch);
+    } else {
+        Launch<MODE, 16>(st, p, batch);
     }
 }
 

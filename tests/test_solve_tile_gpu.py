@@ -72,3 +72,17 @@ def test_inverse_bitwise(handle, n, batch, zero, pivot):
     assert np.array_equal(to_host(info), ginfo)
     assert np.array_equal(got[:, :, :n], gold[:, :, :n], equal_nan=True)
     assert (got[:, :, n:] == 9.0).all()
+
+
+@pytest.mark.parametrize("trans", ["N", "T"])
+@pytest.mark.parametrize("n,nrhs,batch", [(257, 1, 257), (257, 16, 256), (512, 256, 17), (513, 250, 17),
+                                          (1024, 256, 17), (1025, 256, 17)])
+def test_solve_many_units_past_256(handle, trans, n, nrhs, batch):
+    """Orders past 256 with more than 256 units of 16 right-hand sides: four waves a unit to order 512, eight to 1024,
+    sixteen beyond."""
+    test_solve_bitwise(handle, trans, n, nrhs, batch, 0)
+
+
+@pytest.mark.parametrize("n,batch,zero", [(257, 16, 200), (520, 8, None)])
+def test_inverse_many_units_past_256(handle, n, batch, zero):
+    test_inverse_bitwise(handle, n, batch, zero, True)

@@ -1066,22 +1066,27 @@ struct GroupedProblem {
     int slot;               // index into the device pointer arrays (when the launch passes them)
 };
 
-// The problem that holds a tile: the last whose tileStart is at most it.  A
-// wave compares 64 records at a time (one round trip; a binary search's six
-// dependent ones took 6 us before a tile's first load).
+// The problem that holds a tile: the last whose tileStart is at most it
+// (probs[0].tileStart is 0).  A wave compares 64 records at a time, so the
+// search is one round trip up to 64 problems, two to 4096, three to 2^18, where
+// a binary search takes six for 64 (6 us before a tile's first load) and walking
+// the records in order takes count / 64.  FP32, 20000 problems of 64^3: binary
+// 701 us, in order 2318, this 683; 64 problems: 14 us each way.
 __device__ __forceinline__ int ProblemOf(const GroupedProblem* probs, int numProbs, int tile)
 {
-    int last = 0;
-    for (int base = 0; base < numProbs; base += kWaveSize) {
-        const int i = base + (static_cast<int>(threadIdx.x) & 63);
-        const bool before = i < numProbs && dev::G(&probs[min(i, numProbs - 1)].tileStart)[0] <= tile;
-        const int count = __builtin_popcountll(__builtin_amdgcn_ballot_w64(before));
-        last = base + count - 1;
-        if (count < kWaveSize) {
-            break;
-        }
-    }
-    return __builtin_amdgcn_readfirstlane(last);
+    const int lane = static_cast<int>(threadIdx.x) & (kWaveSize - 1);
+    int first = 0;
+    int count = numProbs;
+    int stride;
+    do {
+        stride = (count + kWaveSize - 1) / kWaveSize;
+        const int at = lane * stride;
+        const bool before = at < count && dev::G(&probs[first + min(at, count - 1)].tileStart)[0] <= tile;
+        const int step = (__builtin_popcountll(__builtin_amdgcn_ballot_w64(before)) - 1) * stride;
+        first += step;
+        count = min(stride, count - step);
+    } while (stride > 1);
+    return __builtin_amdgcn_readfirstlane(first);
 }
 
 // L2 group height of the grouped kernel's tile walk (problems are small: a

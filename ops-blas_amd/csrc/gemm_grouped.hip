@@ -438,8 +438,10 @@ extern "C" aclblasStatus_t aclblasGemmGroupedBatchedEx(
             work128 += 1.0 * p.k * tilesOf(p, 128);
         }
     }
+    // 512 threads a tile, and fewer than 2^32 in a launch
+    constexpr long long kMaxDirectTiles = 0x7FFFFF;
     const bool useDirect = handle->tune_override[tune::kOpGrouped][0] == 0 && 2 * direct256 >= cus &&
-                           work256 <= 1.25 * work128;
+                           direct256 <= kMaxDirectTiles && work256 <= 1.25 * work128;
     if (useDirect) {
         std::stable_sort(probs.begin(), probs.end(),
                          [&](const GroupedProblem& x, const GroupedProblem& y) { return part(x) < part(y); });
@@ -459,8 +461,8 @@ extern "C" aclblasStatus_t aclblasGemmGroupedBatchedEx(
         p.tilesN = (p.n + edge - 1) / edge;
         p.tileStart = static_cast<int>(sg.tiles);
         sg.tiles += tilesOf(p, edge);
-        if (sg.tiles > (edge == 256 ? 0x7FFFFFll : 0x7FFFFFFFll)) {
-            LogError("aclblasGemmGroupedBatchedEx", "too many tiles");
+        if (sg.tiles > 0x7FFFFFFFll) {
+            LogError("aclblasGemmGroupedBatchedEx", "more than 2^31 tiles");
             return ACLBLAS_STATUS_NOT_SUPPORTED;
         }
     }

@@ -1,4 +1,4 @@
-"""Grouped GEMM calls of many problems: the search for a tile's problem.
+"""Grouped GEMM calls of many problems (the search for a tile's problem) and of many tiles.
 
 Operands are small integers, so that every product, sum and result is exact: equality with FP64 on the host.
 """
@@ -55,3 +55,32 @@ def test_tile_lookup_over_many_problems(handle, count, dtype):
 def test_tile_lookup_direct_to_lds(handle):
     """Enough 256 x 256 tiles for the direct-to-LDS launch, over 200 problems; every third problem beside it."""
     _run(handle, 300, torch.bfloat16, LARGE)
+
+
+def test_more_tiles_than_a_direct_launch(handle):
+    """One problem wide enough for 2^23 - 1 tiles of 256 columns beside one whose work lets the pair qualify for the
+    direct-to-LDS launch, which cannot hold that many: they take the persistent kernel."""
+    n = 8388607 * 256
+    big = 16384
+    a = torch.ones(8, 8, dtype=torch.bfloat16, device="cuda")
+    b = torch.ones(n, 8, dtype=torch.bfloat16, device="cuda")
+    c = torch.zeros(n, 8, dtype=torch.bfloat16, device="cuda")
+    a2 = torch.zeros(2 * big, big, dtype=torch.bfloat16, device="cuda")
+    a2[0] = 1.0
+    b2 = torch.zeros(big, 2 * big, dtype=torch.bfloat16, device="cuda")
+    b2[:, 0] = torch.arange(big, device="cuda") % 256
+    c2 = torch.zeros(big, big, dtype=torch.bfloat16, device="cuda")
+    pa, pb, pc = (torch.tensor([x.data_ptr(), y.data_ptr()], dtype=torch.int64, device="cuda")
+                  for x, y in ((a, a2), (b, b2), (c, c2)))
+    st = B.gemm_grouped_batched_ex(handle.value, [B.OP_N] * 2, [B.OP_N] * 2, [8, big], [n, big], [8, 2 * big],
+                                   [1.0] * 2, pa.data_ptr(), B.ACL_BF16, [8, big], pb.data_ptr(), B.ACL_BF16,
+                                   [8, 2 * big], [0.0] * 2, pc.data_ptr(), B.ACL_BF16, [8, big], [1] * 2,
+                                   B.COMPUTE["COMPUTE_32F"])
+    assert st == 0, st
+    torch.cuda.synchronize()
+    for at in range(0, n, 1 << 28):
+        assert bool((c[at:at + (1 << 28)] == 8.0).all()), at
+    want = (torch.arange(big, device="cuda") % 256).to(torch.bfloat16)
+    assert torch.equal(c2, want[:, None].expand(big, big))
+    del a, b, c, a2, b2, c2
+    torch.cuda.empty_cache()

@@ -240,3 +240,31 @@ def test_mx_tiles_agree(lt, fp4, trans, m, n):
                             sa, sw, None, c1 - c0, c1 - c0)
             assert st == 0
             assert np.array_equal(full[r0:r1, c0:c1], part)
+
+
+@pytest.mark.parametrize("fp4", [False, True], ids=["mxfp8", "mxfp4"])
+@pytest.mark.parametrize("trans", ["NN", "NT", "TN", "TT"])
+def test_mx_register_staged_tiles_agree(lt, fp4, trans):
+    """Rows of both operands padded to pitches that are no multiple of 16 bytes, odd m and n, a last K block alone in
+    its stage, zero scale bytes, and 289 tiles of 128: the register-staged kernel with its larger tile gives the bits
+    of the smallest one on corner blocks."""
+    rng = np.random.default_rng(911 + fp4)
+    m, n, k, (ta, tb) = 2049, 2083, 416, trans
+    typ = O.LT_MXFP4 if fp4 else O.LT_MXFP8
+    A, lda = _mx_operand(rng, *((m, k + 6) if ta == "N" else (k, m + 6)), fp4)
+    W, ldb = _mx_operand(rng, *((k, n + 6) if tb == "N" else (n, k + 6)), fp4)
+    assert lda % 16 and ldb % 16
+    sA = rng.integers(120, 135, size=_scale_bytes(m, k, ta != "N")).astype(np.uint8)
+    sW = rng.integers(120, 135, size=_scale_bytes(n, k, tb == "N")).astype(np.uint8)
+    sA[rng.integers(0, sA.size, 4000)] = 0
+    sW[rng.integers(0, sW.size, 4000)] = 0
+    st, full = _run(lt, typ, B.ACL_FLOAT, ta, tb, m, n, k, 1.0, 0.0, A, lda, W, ldb, sA, sW, None, n, n)
+    assert st == 0
+    for r0, r1 in ((0, 62), (1000, 1064), (m // 2 * 2 - 64, m)):
+        for c0, c1 in ((0, 60), (1020, 1084), (n // 2 * 2 - 62, n)):
+            a, sa = _mx_slice(A, sA, fp4, m, k, ta == "T", r0, r1)
+            w, sw = _mx_slice(W, sW, fp4, n, k, tb == "N", c0, c1)
+            st, part = _run(lt, typ, B.ACL_FLOAT, ta, tb, r1 - r0, c1 - c0, k, 1.0, 0.0, a, a.shape[1], w, w.shape[1],
+                            sa, sw, None, c1 - c0, c1 - c0)
+            assert st == 0
+            assert np.array_equal(full[r0:r1, c0:c1], part)

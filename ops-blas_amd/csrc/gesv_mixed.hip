@@ -957,6 +957,10 @@ extern "C" aclblasStatus_t aclblasSgesvBatchedMixedEx(
     // per call in one launch per stage / in parts: BF16X2 10000 systems 5102 /
     // 5022, 2800 1710 / 1674, 2200 1327 / 1384 (so not split); FP32 8000 systems
     // 3900 / 3670, 3300 1901 / 1711, 2500 1423 / 1472 (not split).
+    // The one- and three-plane updates send systems to the FP32 pass and to
+    // more corrections, whose stragglers end each launch: kept in one unless all
+    // orders are small (3000 systems, one / in parts: BF16 3915 / 4229, BF16X3
+    // 3464 / 3909).
     const auto above = [&](int n) {
         return static_cast<int>(
             std::partition_point(table.begin(), table.end(), [n](const MixedSystem& s) { return s.n > n; }) -
@@ -965,7 +969,8 @@ extern "C" aclblasStatus_t aclblasSgesvBatchedMixedEx(
     const auto fills = [&](int first, int last, int perCu) { return last - first >= perCu * cus; };
     const int n128 = above(kSmallN);
     const int n192 = above(kMidN);
-    const bool split = fills(n128, batchCount, 5) && (n128 == 0 || fills(0, n128, 5));
+    const bool even = mode == ACLBLAS_MIXED_UPDATE_FP32 || mode == ACLBLAS_MIXED_UPDATE_BF16X2;
+    const bool split = fills(n128, batchCount, 5) && (n128 == 0 || (even && fills(0, n128, 5)));
     const int smallFrom = split ? n128 : batchCount;
     MarkLaunch(handle, 0);
     if (split && mode == ACLBLAS_MIXED_UPDATE_FP32) {

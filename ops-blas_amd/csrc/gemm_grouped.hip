@@ -417,7 +417,8 @@ extern "C" aclblasStatus_t aclblasGemmGroupedBatchedEx(
     // direct-to-LDS kernel, one launch per transpose pair, when their 256 tiles
     // occupy half the CUs or more and pad the work by at most a quarter over 128
     // tiles; the rest to the persistent kernel.  64 shapes up to 2048 (padding
-    // 1.12) 557 -> 384 us; 64 shapes up to 512 (1.39) would take 45 instead of 39.
+    // 1.09) take 514 us there and 385 here, up to 1024 (1.20) 100 and 85; up to 512
+    // (1.27 to 1.35) 35 and 43.
     // A launch choice forced on the handle keeps the persistent kernel.
     const bool sixteen = Atype == ACL_FLOAT16 || Atype == ACL_BF16;
     const auto part = [&](const GroupedProblem& p) {

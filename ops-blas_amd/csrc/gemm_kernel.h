@@ -154,9 +154,9 @@ struct TileLoader {
 
     // Sixteen bytes at any alignment the element type allows (the hardware's
     // global loads take any address): operands whose base or leading dimension
-    // is not a multiple of 16 bytes used to be read element by element, 4 times
-    // slower over a ragged 16-bit group (64 odd shapes up to 2048: 2320 us, 775 us
-    // now).
+    // is not a multiple of 16 bytes used to be read element by element, three
+    // times slower over a ragged 16-bit group (64 odd shapes up to 2048: 2729 us,
+    // 956 us now).
     __device__ __forceinline__ static uint4 LoadAny(const uint8_t* p)
     {
         const auto v = *(const ACL_GLOBAL U32x4Any*)p;
@@ -1166,7 +1166,10 @@ inline void LaunchGemmTyped(hipStream_t st, GemmArgs p, int batch, int tile, int
     p.group = group;
     if constexpr (KA == kBF16 || KA == kF16) {
         // direct-to-LDS kernel: 16-byte aligned operands (a batch's pointers are
-        // checked on the device), and an index-contiguous operand's extent a
+        // checked on the device; a problem whose pointers are not loads its stages
+        // through registers there, no slower than the register-staged kernel: 64
+        // products of 512^3, NN, A 8 bytes off 37 us, there with a padded leading
+        // dimension 39, aligned 29), and an index-contiguous operand's extent a
         // whole number of 16-byte chunks (its DMA copies whole chunks: a partial
         // last chunk would read past the end of the operand's last column)
         if (tile == 256 && p.vecA != 0 && p.vecB != 0 && DmaExtentsWhole(p, 8)) {

@@ -153,10 +153,6 @@ struct RefineShared {
 
 __device__ __forceinline__ double MaxD(double a, double b) { return b > a ? b : a; }
 
-// ok ? p[idx] : 0 with an unconditional load (of p[0] when !ok, which is in
-// bounds wherever this is used): the compiler can then issue the loads of a
-// sequence together, where a load under a lane-dependent condition is issued
-// inside a branch and waited for there.
 // The pointer, made opaque to the optimiser at this point: addresses derived
 // from it are computed here instead of being hoisted out of the enclosing
 // refinement loop, where they would stay live across the solves and spill.
@@ -173,6 +169,10 @@ __device__ __forceinline__ T* Opaque(T* p)
 // its first use and waits for it there).
 __device__ __forceinline__ void LoadsBeforeUses() { __builtin_amdgcn_sched_barrier(0); }
 
+// ok ? p[idx] : 0 with an unconditional load (of p[0] when !ok, which is in
+// bounds wherever this is used): the compiler can then issue the loads of a
+// sequence together, where a load under a lane-dependent condition is issued
+// inside a branch and waited for there.
 template <typename T, typename P>
 __device__ __forceinline__ T LoadOr0(P p, size_t idx, bool ok)
 {
@@ -242,8 +242,11 @@ __device__ __forceinline__ void BackSubstituteAny(float (&x)[R], const float (&u
 // before it is worked on, and the barriers wait for LDS only, so the loads stay
 // in flight across them; before, each panel paid a memory round trip for the
 // map, the inverse and the block in turn, and the substitution ran its
-// right-hand sides one after the other, a division each (refine of 10000
-// systems of order 16..256, two-plane updates: 2.86 -> 2.36 ms).
+// right-hand sides one after the other, a division each (the refine kernels of
+// 10000 systems of order 16..256, two-plane updates: 2.57 -> 2.07 ms with the
+// instance for orders up to 128).  The operands in flight take registers that
+// three waves a SIMD do not leave: 224 bytes a lane of either instance live in
+// scratch.  Needs n >= 1: the prefetches run before the loops' bounds.
 template <int N>
 __device__ __forceinline__ void FactoredSolve(const MixedSystem& s, RefineShared<N>& sh)
 {
@@ -951,8 +954,8 @@ extern "C" aclblasStatus_t aclblasSgesvBatchedMixedEx(
     // solve up to kSmallN (six two-wave workgroups per CU for three of four
     // waves, whose upper two have no rows there) and, with FP32 updates, the
     // factorisation up to kSmallN and kMidN (four and three workgroups per CU
-    // for two; the BF16 instances are at three already and gained nothing from a
-    // fourth).  Only when each part fills the card several times: the next
+    // for two, at the price of 68 bytes a lane in scratch up to kSmallN; the BF16
+    // instances are at three already and gained nothing from a fourth).  Only when each part fills the card several times: the next
     // launch waits for the last systems of the one before.  Orders 16..256, us
     // per call in one launch per stage / in parts: BF16X2 10000 systems 5102 /
     // 5022, 2800 1710 / 1674, 2200 1327 / 1384 (so not split); FP32 8000 systems

@@ -130,7 +130,8 @@ void LaunchGetrfBlocked(hipStream_t st, float* const* A, int n, int lda, int* ip
     // leave a CU idle, so the instance for the order at hand (less LDS, fewer
     // accumulators) puts more workgroups on it.  2048 x 128: 590 us with the
     // 256 instance (two per CU, left columns permuted one at a time), 445 us
-    // with three per CU, 370 us with four.
+    // with three per CU, 360 us with four, although 156 bytes a lane then live in
+    // scratch.
     if (n <= 128) {
         Launch<PIVOT, 128, 4>(st, A, n, lda, ipiv, info, batch, cus);
     } else if (n <= 192) {

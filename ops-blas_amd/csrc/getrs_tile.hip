@@ -23,9 +23,9 @@
 // The kernel before it solved 64-row blocks with one row per lane (a division
 // and a broadcast per right-hand side and step) and built the row permutation
 // with one thread.  Measured before and now:
-//   2048 systems of order 128, 8 right-hand sides: N 277 -> 66 us, T 283 -> 74 us
+//   2048 systems of order 128, 8 right-hand sides: N 277 -> 65 us, T 283 -> 74 us
 //   inverse of 500 matrices of order 100: 717 -> 103 us
-//   8 systems of order 1000, 4 right-hand sides, T: 1040 -> 390 us
+//   8 systems of order 1000, 4 right-hand sides, T: 1095 -> 378 us
 #include "device_common.h"
 #include "internal.h"
 #include "lapack_kernels.h"
@@ -468,12 +468,15 @@ __device__ __forceinline__ void SolveAlone(const Tiles<LOWER, TR>& T, float (*di
 
 // Bytes of LDS of one (system, 16 right-hand sides): unknowns, permutation and
 // the traced sources of its swap groups.
-__host__ __device__ inline int UnitBytes(int n)
+__host__ __device__ constexpr int UnitBytes(int n)
 {
     const int tiles = (n + kT - 1) / kT;
     const int groups = (n + kSwaps - 1) / kSwaps;
     return tiles * kT * kT * 4 + (((n + 7) & ~7) + groups * 2 * kSwaps) * 2;
 }
+constexpr int kDiagBytes = 4 * kT * (kT + 4) * 4;  // the diagonal blocks beside the units
+static_assert(UnitBytes(kMaxTileN) + kDiagBytes <= 160 * 1024, "a unit of the largest order fits in LDS");
+static_assert(4 * UnitBytes(256) + kDiagBytes <= 160 * 1024, "four units of one wave each fit in LDS");
 
 // Unit u = (system u / chunks, chunk u % chunks of 16 right-hand sides).
 // WAVES > 1: one unit per workgroup of WAVES waves.  WAVES == 1: one per wave,

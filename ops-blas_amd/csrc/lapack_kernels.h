@@ -31,7 +31,8 @@ bool LaunchGetrsSmall(hipStream_t st, bool trans, int n, int nrhs, const float* 
 
 // Triangular solves (op N / T) and inverses of orders 65..kMaxTileN, 16
 // right-hand sides per workgroup (getrs_tile.hip); the bound is the tiles'
-// LDS: 64 bytes per row and 12 for the permutation, 152 KiB at 2048.
+// LDS: 64 bytes per row, 6 for the permutation and 5 KiB of diagonal blocks, 145
+// of the 160 KiB at 2048.
 constexpr int kMaxTileN = 2048;
 enum SolveTileMode { kSolveN = 0, kSolveT = 1, kSolveInv = 2 };
 template <SolveTileMode MODE>

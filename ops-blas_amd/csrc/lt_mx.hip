@@ -38,10 +38,12 @@
 // What bounds it: the LDS round trips at the start of a stage (its fragments
 // can only be read after the barrier) against 32 matrix instructions per wave
 // with 256 x 256 tiles and 16 with 128 x 128; the larger tile, whose two waves
-// per SIMD also cover for each other, reaches 1.6 PFLOP/s.  4096^3, BF16 out, A
-// and B K-contiguous (NT) / both row-contiguous (TN): MXFP8 332 -> 84 / 2490
-// -> 88 us, MXFP4 191 -> 76 / 1523 -> 62 us (before: 64 x 64 tiles, element-wise
-// transposes, no load in flight during the products).  Fragments of the next
+// per SIMD also cover for each other, reaches 1.6 PFLOP/s (MXFP8: matrix cores
+// busy a third of the time; 24 to 92 bytes a lane of that instance live in
+// scratch).  4096^3, BF16 out, A and B K-contiguous (NT) / both row-contiguous
+// (TN): MXFP8 329 -> 90 / 2537 -> 77 us, MXFP4 176 -> 67 / 1522 -> 55 us (before:
+// 64 x 64 tiles, element-wise transposes, no load in flight during the
+// products).  Fragments of the next
 // stage held in registers during the products were slower (174 us: the
 // compiler moves them through the accumulation registers).
 #include <hip/hip_runtime.h>
@@ -681,8 +683,9 @@ void Launch(hipStream_t st, MxArgs p)
 {
     // Largest tiles that still give (about) every CU one: larger tiles need
     // fewer LDS bytes per product, fewer tiles leave CUs idle.  MXFP8 NT: 4096^3
-    // 84 us with 256 tiles (156 with 128); 2048^3 54 us with 256 and 29 with
-    // 128 tiles; 1024 x 1024 x 4096 37 us with 128 and 20 with 64.
+    // 92 us with 256 tiles (143 with 128); 2048^3 46 us with 256 and 23 with 128
+    // tiles; 1024 x 1024 x 4096 36 us with 128 and 17 with 64.  (3072^3, 144 tiles
+    // of 256, takes 84 us with 128 tiles and would take 64 with 256.)
     const auto tiles = [&](int bt) {
         p.tilesM = (p.m + bt - 1) / bt;
         p.tilesN = (p.n + bt - 1) / bt;

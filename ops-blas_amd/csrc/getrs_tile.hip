@@ -1,6 +1,6 @@
 // Triangular solves and inverses with the LU factors of orders 65..2048:
-// one workgroup per (system, 16 right-hand sides), the unknowns as 16 x 16
-// tiles in LDS, everything off the diagonal blocks on the FP32 matrix
+// one workgroup per unit of a system and 16 (or, of many, 4) right-hand sides, the
+// unknowns as 16 x 16 tiles in LDS, everything off the diagonal blocks on the FP32 matrix
 // instruction.
 //
 // Reference: blas/getrs_batched/arch35/sgetrs_batched_kernel.cpp:83-410 (N: P,
@@ -37,18 +37,26 @@ namespace {
 
 using dev::kWave;
 
-constexpr int kT = 16;        // tile order and right-hand sides per workgroup
+constexpr int kT = 16;        // tile order, and most right-hand sides of a unit
+constexpr int kFew = 4;       // right-hand sides of a narrow unit
 constexpr int kSwaps = 64;    // interchanges composed per step of the permutation
 constexpr int kAheadTiles = 4;  // tiles of a wave whose operands are loaded a phase ahead
 
 using f32x4 = dev::F32x4;
 
-// Unknown (row, rhs) in LDS: rows of 16, each quad of rows rotated by its own
-// number, so that both a quarter-wave's four consecutive rows (matrix operand)
-// and rows four apart (accumulators) fall into distinct banks.
+// Unknown (row, rhs) in LDS.  COLS 16: rows of 16, each quad of rows rotated by
+// its own number, so that both a quarter-wave's four consecutive rows (matrix
+// operand) and rows four apart (accumulators) fall into distinct banks.  COLS
+// 4: rows of 4, conflict-free in order; lanes past the fourth column repeat the
+// first four.
+template <int COLS>
 __device__ __forceinline__ int XOff(int row, int rhs)
 {
-    return ((row & ~3) + ((row + (row >> 2)) & 3)) * kT + rhs;
+    if constexpr (COLS == kT) {
+        return ((row & ~3) + ((row + (row >> 2)) & 3)) * kT + rhs;
+    } else {
+        return row * COLS + (rhs & (COLS - 1));
+    }
 }
 
 // Makes LDS writes of the WAVES waves that work together visible to them.
@@ -231,7 +239,7 @@ __device__ __forceinline__ void TransposeGroups(f32x4& v)
 // 16-byte aligned and whole tiles are read with one 16-byte load per lane
 // (four consecutive columns of op, put into chain order by a 4 x 4 transpose
 // between lane groups).
-template <bool LOWER, bool TR>
+template <bool LOWER, bool TR, int COLS>
 struct Tiles {
     const float* Aptr;
     size_t ld;
@@ -299,7 +307,7 @@ struct Tiles {
         f32x4 x;
         dev::StaticFor<0, 4>([&](auto jc) {
             constexpr int j = decltype(jc)::value;
-            x[j] = xs[XOff(kT * I + 4 * grp + j, r16)];
+            x[j] = xs[XOff<COLS>(kT * I + 4 * grp + j, r16)];
         });
         return x;
     }
@@ -309,7 +317,7 @@ struct Tiles {
             constexpr int j = decltype(jc)::value;
             const int row = kT * I + 4 * grp + j;
             if (row < n) {
-                xs[XOff(row, r16)] = x[j];  // rows past the order stay +0
+                xs[XOff<COLS>(row, r16)] = x[j];  // rows past the order stay +0
             }
         });
     }
@@ -319,7 +327,7 @@ struct Tiles {
         f32x4 v;
         dev::StaticFor<0, 4>([&](auto sc) {
             constexpr int s = decltype(sc)::value;
-            v[s] = xs[XOff(Column(P, s), r16)];
+            v[s] = xs[XOff<COLS>(Column(P, s), r16)];
         });
         return v;
     }
@@ -349,8 +357,8 @@ __device__ __forceinline__ void Chain(const f32x4& a, const f32x4& b, f32x4& x)
 
 // One triangular solve by the workgroup: in phase J the wave that owns tile J
 // updates and solves it first, the others apply X(J-1) to the tiles behind it.
-template <bool LOWER, bool UNIT, bool TR, int WAVES>
-__device__ __forceinline__ void SolveShared(const Tiles<LOWER, TR>& T, int wave, float (*diag)[kT][kT + 4])
+template <bool LOWER, bool UNIT, bool TR, int WAVES, int COLS>
+__device__ __forceinline__ void SolveShared(const Tiles<LOWER, TR, COLS>& T, int wave, float (*diag)[kT][kT + 4])
 {
     const int nt = T.nt;
     f32x4 nextOp{};
@@ -426,7 +434,7 @@ __device__ __forceinline__ void SolveShared(const Tiles<LOWER, TR>& T, int wave,
 // before it, then its diagonal block; the operands of tile J + 1 are loaded
 // while the block of tile J is solved.
 template <bool LOWER, bool UNIT, bool TR>
-__device__ __forceinline__ void SolveAlone(const Tiles<LOWER, TR>& T, float (*diag)[kT + 4])
+__device__ __forceinline__ void SolveAlone(const Tiles<LOWER, TR, kT>& T, float (*diag)[kT + 4])
 {
     constexpr int kRun = 8;
     f32x4 ops[kRun] = {};
@@ -466,23 +474,23 @@ __device__ __forceinline__ void SolveAlone(const Tiles<LOWER, TR>& T, float (*di
     }
 }
 
-// Bytes of LDS of one (system, 16 right-hand sides): unknowns, permutation and
-// the traced sources of its swap groups.
-__host__ __device__ constexpr int UnitBytes(int n)
+// Bytes of LDS of one unit (system, cols right-hand sides): unknowns,
+// permutation and the traced sources of its swap groups.
+__host__ __device__ constexpr int UnitBytes(int n, int cols)
 {
     const int tiles = (n + kT - 1) / kT;
     const int groups = (n + kSwaps - 1) / kSwaps;
-    return tiles * kT * kT * 4 + (((n + 7) & ~7) + groups * 2 * kSwaps) * 2;
+    return tiles * kT * cols * 4 + (((n + 7) & ~7) + groups * 2 * kSwaps) * 2;
 }
 constexpr int kDiagBytes = 4 * kT * (kT + 4) * 4;  // the diagonal blocks beside the units
-static_assert(UnitBytes(kMaxTileN) + kDiagBytes <= 160 * 1024, "a unit of the largest order fits in LDS");
-static_assert(4 * UnitBytes(256) + kDiagBytes <= 160 * 1024, "four units of one wave each fit in LDS");
+static_assert(UnitBytes(kMaxTileN, kT) + kDiagBytes <= 160 * 1024, "a unit of the largest order fits in LDS");
+static_assert(4 * UnitBytes(256, kT) + kDiagBytes <= 160 * 1024, "four units of one wave each fit in LDS");
 
-// Unit u = (system u / chunks, chunk u % chunks of 16 right-hand sides).
+// Unit u = (system u / chunks, chunk u % chunks of COLS right-hand sides).
 // WAVES > 1: one unit per workgroup of WAVES waves.  WAVES == 1: one per wave,
 // four waves per workgroup that never wait for each other.
 // kSolveInv: C = A^-1 out of place (B = C), nrhs = n, info written per matrix.
-template <SolveTileMode MODE, int WAVES>
+template <SolveTileMode MODE, int WAVES, int COLS>
 __global__ __launch_bounds__(WAVES == 1 ? 4 * kWave : WAVES * kWave) void SolveTileKernel(SolveTileArgs p)
 {
     constexpr int kUnits = WAVES == 1 ? 4 : 1;
@@ -496,15 +504,15 @@ __global__ __launch_bounds__(WAVES == 1 ? 4 * kWave : WAVES * kWave) void SolveT
     if (unit >= p.units) {
         return;  // a wave of its own: nobody waits for it
     }
-    uint8_t* const mem = smem + (WAVES == 1 ? group * UnitBytes(n) : 0);
+    uint8_t* const mem = smem + (WAVES == 1 ? group * UnitBytes(n, COLS) : 0);
     float* xs = reinterpret_cast<float*>(mem);
-    uint16_t* perm = reinterpret_cast<uint16_t*>(xs + nt * kT * kT);
+    uint16_t* perm = reinterpret_cast<uint16_t*>(xs + nt * kT * COLS);
     uint16_t* from = perm + ((n + 7) & ~7);
 
     const int b = static_cast<int>(unit / p.chunks);
     const int chunk = static_cast<int>(unit - static_cast<long long>(b) * p.chunks);
-    const int r0 = chunk * kT;
-    const int rc = min(kT, p.nrhs - r0);
+    const int r0 = chunk * COLS;
+    const int rc = min(COLS, p.nrhs - r0);
     const float* A = p.A[b];
     const auto B = dev::G(p.B[b]);
     const int t = wave * kWave + dev::LaneId();
@@ -516,8 +524,8 @@ __global__ __launch_bounds__(WAVES == 1 ? 4 * kWave : WAVES * kWave) void SolveT
     // rows permuted for the N and inverse solves; rows and columns past the ends are +0
     for (int i = t; i < nt * kT; i += kThreads) {
         const int src = MODE != kSolveT && i < n ? permOf(i) : i;
-        float v[kT];
-        dev::StaticFor<0, kT>([&](auto rcst) {
+        float v[COLS];
+        dev::StaticFor<0, COLS>([&](auto rcst) {
             constexpr int r = decltype(rcst)::value;
             if (MODE == kSolveInv) {
                 v[r] = i < n && src == r0 + r ? 1.0f : 0.0f;
@@ -525,9 +533,9 @@ __global__ __launch_bounds__(WAVES == 1 ? 4 * kWave : WAVES * kWave) void SolveT
                 v[r] = i < n && r < rc ? B[src + static_cast<size_t>(r0 + r) * p.ldb] : 0.0f;
             }
         });
-        dev::StaticFor<0, kT>([&](auto rcst) {
+        dev::StaticFor<0, COLS>([&](auto rcst) {
             constexpr int r = decltype(rcst)::value;
-            xs[XOff(i, r)] = v[r];
+            xs[XOff<COLS>(i, r)] = v[r];
         });
     }
     Sync<WAVES>();
@@ -536,11 +544,11 @@ __global__ __launch_bounds__(WAVES == 1 ? 4 * kWave : WAVES * kWave) void SolveT
         constexpr bool kLower = decltype(lower)::value;
         constexpr bool kUnit = decltype(unitDiag)::value;
         constexpr bool kTr = decltype(tr)::value;
-        const Tiles<kLower, kTr> T(A, p.lda, n, vec, xs);
+        const Tiles<kLower, kTr, COLS> T(A, p.lda, n, vec, xs);
         if constexpr (WAVES == 1) {
             SolveAlone<kLower, kUnit, kTr>(T, diag[group]);
         } else {
-            SolveShared<kLower, kUnit, kTr, WAVES>(T, wave, diag);
+            SolveShared<kLower, kUnit, kTr, WAVES, COLS>(T, wave, diag);
         }
     };
     if constexpr (MODE == kSolveT) {
@@ -567,20 +575,20 @@ __global__ __launch_bounds__(WAVES == 1 ? 4 * kWave : WAVES * kWave) void SolveT
     }
     for (int i = t; i < n; i += kThreads) {
         const int row = MODE == kSolveT ? permOf(i) : i;
-        dev::StaticFor<0, kT>([&](auto rcst) {
+        dev::StaticFor<0, COLS>([&](auto rcst) {
             constexpr int r = decltype(rcst)::value;
             if (r < rc) {
-                B[row + static_cast<size_t>(r0 + r) * p.ldb] = xs[XOff(i, r)];
+                B[row + static_cast<size_t>(r0 + r) * p.ldb] = xs[XOff<COLS>(i, r)];
             }
         });
     }
 }
 
-template <SolveTileMode MODE, int WAVES>
+template <SolveTileMode MODE, int WAVES, int COLS = kT>
 void Launch(hipStream_t st, const SolveTileArgs& p, int batch)
 {
     constexpr int kUnits = WAVES == 1 ? 4 : 1;
-    const size_t lds = static_cast<size_t>(UnitBytes(p.n)) * kUnits;
+    const size_t lds = static_cast<size_t>(UnitBytes(p.n, COLS)) * kUnits;
     // slices keep a launch's threads below 2^32
     const int slice = (1 << 21) / p.chunks;
     for (int b0 = 0; b0 < batch; b0 += slice) {
@@ -591,9 +599,27 @@ void Launch(hipStream_t st, const SolveTileArgs& p, int batch)
         q.ipiv = p.ipiv != nullptr ? p.ipiv + static_cast<size_t>(b0) * p.n : nullptr;
         q.info = p.info != nullptr ? p.info + b0 : nullptr;
         q.units = static_cast<long long>(count) * p.chunks;
-        hipLaunchKernelGGL((SolveTileKernel<MODE, WAVES>), dim3(static_cast<unsigned>((q.units + kUnits - 1) / kUnits)),
+        hipLaunchKernelGGL((SolveTileKernel<MODE, WAVES, COLS>),
+                           dim3(static_cast<unsigned>((q.units + kUnits - 1) / kUnits)),
                            dim3(WAVES == 1 ? 4 * kWave : WAVES * kWave), lds, st, q);
     }
+}
+
+// Many units past order 256: up to four right-hand sides in units of four
+// columns, whose LDS is a quarter, so that the registers bound the units on a
+// CU and not the LDS.  N, 1 right-hand side, us with sixteen / four columns:
+// order 512, 1200 systems 426 / 337; order 700, 1000 systems 613 / 552, 1200 768
+// / 646 (the row-per-lane kernel before these: 386, 593 and 648).
+template <SolveTileMode MODE, int WAVES>
+void LaunchFew(hipStream_t st, const SolveTileArgs& p, int batch)
+{
+    if constexpr (MODE != kSolveInv) {
+        if (p.nrhs <= kFew) {
+            Launch<MODE, WAVES, kFew>(st, p, batch);
+            return;
+        }
+    }
+    Launch<MODE, WAVES>(st, p, batch);
 }
 
 }  // namespace
@@ -614,7 +640,7 @@ void LaunchSolveTile(hipStream_t st, int n, int nrhs, const float* const* A, int
     // it.  N, 1 right-hand side, us with 16 / 8 / 4 waves: order 257, 256 systems
     // 64 / 67 / 74, 2000 systems 510 / 327 / 229; order 700, 256 systems 205 /
     // 224 / 327, 1000 systems 823 / 615 / 772; order 1200, 300 systems 861 /
-    // 1063 / 1819.
+    // 1063 / 1819.  Up to four right-hand sides these take units of four columns.
     if (n <= 256) {
         if (units >= 1536) {
             Launch<MODE, 1>(st, p, batch);
@@ -622,9 +648,9 @@ void LaunchSolveTile(hipStream_t st, int n, int nrhs, const float* const* A, int
             Launch<MODE, 4>(st, p, batch);
         }
     } else if (units > 256 && n <= 512) {
-        Launch<MODE, 4>(st, p, batch);
+        LaunchFew<MODE, 4>(st, p, batch);
     } else if (units > 256 && n <= 1024) {
-        Launch<MODE, 8>(st, p, batch);
+        LaunchFew<MODE, 8>(st, p, batch);
     } else {
         Launch<MODE, 16>(st, p, batch);
     }

@@ -83,6 +83,14 @@ def test_solve_many_units_past_256(handle, trans, n, nrhs, batch):
     test_solve_bitwise(handle, trans, n, nrhs, batch, 0)
 
 
+@pytest.mark.parametrize("trans", ["N", "T"])
+@pytest.mark.parametrize("n,nrhs,batch", [(257, 1, 300), (300, 4, 257), (300, 5, 257), (512, 2, 257), (513, 3, 257),
+                                          (1000, 1, 257), (1024, 4, 257), (1025, 4, 257)])
+def test_solve_many_units_of_few_right_hand_sides(handle, trans, n, nrhs, batch):
+    """Up to four right-hand sides of many systems past order 256 run in units of four columns."""
+    test_solve_bitwise(handle, trans, n, nrhs, batch, 0)
+
+
 @pytest.mark.parametrize("n,batch,zero", [(257, 16, 200), (520, 8, None)])
 def test_inverse_many_units_past_256(handle, n, batch, zero):
     test_inverse_bitwise(handle, n, batch, zero, True)
